@@ -389,20 +389,17 @@ struct Workspace {
 // ranges against long key ranges: decode, last-window scoring), each row
 // block's key tiles are dealt to nsplit workgroups of at least 8 tiles,
 // aiming at ~512 workgroups in all.  Depends on sizes only, so the workspace
-// query and the launch agree.  The scores variant splits only up to 64 row
-// blocks, 128 when the key range is at least 8 times the query range, 256
-// at 64 times: its split route writes the scores in a second kernel, which
-// the fused writer beats while it still has a quarter of the CUs busy, or
-// half or all of them over keys not much longer than its rows (B2 H32 M512
-// N16384: 0.607 against 0.734 ms fused; B1 H32 M1024 N16384: 0.547 against
-// 0.592; B8 H32 M256 N16384: 1.27 against 1.58; but B4 H32 M512 N16384:
-// 1.19 against 1.16 fused; B1 H32 M = N = 1024 stays fused).
-constexpr int64_t kScoresSplitMaxWgs = 64;
+// query and the launch agree.  The scores variant writes its scores in a second kernel on this
+// route, so it splits only where the fused writer keeps few CUs busy for
+// long: up to 32 row blocks from 2048 keys on when the key range is at least
+// twice the query range (us, split against fused, B1 D128 causal: H4 M2048
+// N4096 57 / 67; H1 M1024 N2048 41 / 37; H12 M1024 N1024 44 / 24; H4 M256
+// N1024 36 / 23), up to 128 at 8 times (B2 H32 M512 N16384 607 / 734; H12
+// M1024 N4096 96 / 68), and up to 256 at 64 times (B8 H32 M256 N16384 1270 /
+// 1580).
 static int64_t scores_split_max_wgs(const Problem& pr) {
-  const int64_t m = pr.M;
-  return pr.N >= 64 * m ? 4 * kScoresSplitMaxWgs
-         : pr.N >= 8 * m ? 2 * kScoresSplitMaxWgs
-                         : kScoresSplitMaxWgs;
+  const int64_t m = pr.M, n = pr.N;
+  return n >= 64 * m ? 256 : n >= 8 * m ? 128 : n >= 2 * m && n >= 2048 ? 32 : 0;
 }
 // Bytes of the fp32 partials of a plan (O, offset, weight sum, row sum).
 size_t split_bytes(const Problem& pr, const SplitPlan& sp) {
@@ -890,6 +887,14 @@ static int check_scores_out(const char* fn, const void* scores, const int64_t* s
   return FAS_OK;
 }
 
+// Whether every score row starts on a 64-byte boundary (and ends on a 16-byte
+// one): the kernels then stream whole half-lines past the caches, otherwise
+// through them (store_score16 has both sides measured).
+static int score_rows_aligned(const void* scores, const int64_t* st, int64_t n) {
+  return (reinterpret_cast<uintptr_t>(scores) & 63u) == 0 && st[0] % 32 == 0 && st[1] % 32 == 0 &&
+         st[2] % 32 == 0 && n % 8 == 0;
+}
+
 // Scores alone through the scores-only kernel; mask selects the causal /
 // key-range mask with masked entries written as 0.
 static int run_scores(const char* fn, const fas_attn_args* a, const Problem& pr, void* scores,
@@ -919,17 +924,13 @@ static int run_scores(const char* fn, const fas_attn_args* a, const Problem& pr,
     p.spr = (int)((steps + nrs - 1) / nrs);
     p.nrs = (int)((steps + p.spr - 1) / p.spr);
   }
-  p.vec = aligned16(scores) && st[0] % 8 == 0 && st[1] % 8 == 0 && st[2] % 8 == 0 &&
-                  pr.N % 8 == 0
-              ? 1
-              : 0;
-  // Up to 512 query rows with 16-byte score stores: the resident-Q kernel,
-  // one workgroup per CU, each walking two or more of its head's 512-key
-  // blocks.
+  p.aligned = score_rows_aligned(scores, st, pr.N);
+  // Up to 512 query rows: the resident-Q kernel, one workgroup per CU, each
+  // walking two or more of its head's 512-key blocks.
   // Under GQA a workgroup takes the largest power-of-two share of a KV
   // head's query heads whose rows fit (K loaded once for all of them), as
   // long as its q and score offsets stay 31-bit.
-  if (p.vec && pr.M <= fas::kScoresResidentRows) {
+  if (pr.M <= fas::kScoresResidentRows) {
     const int64_t nkb = (pr.N + fas::kScoresResidentKeys - 1) / fas::kScoresResidentKeys;
     int pshift = 0;
     auto fits = [&](int pk) {
@@ -983,40 +984,47 @@ static int attention_with_scores_impl(const fas_attn_args* a, void* scores, cons
       ((pw.pack != 2 && pw.pack != 4 && pw.pack != 8) ||
        ((int64_t)(pw.pack - 1) * st[1] + (int64_t)(bm / pw.pack + 2) * st[2]) * 2 >= kMaxSliceBytes))
     pw.pack = 1;
-  // One workgroup runs per CU.  When 256-row blocks would all run in one
-  // round (the longest causal row block is then the critical path), unpacked
-  // launches take 128-row blocks (4 waves): twice the workgroups, in two
-  // rounds the mirror order balances (B1 H32 S1024: 45.7 -> 37.5 us; H16
-  // S4096: 179 -> 145 us; H32 S2048: 94.3 -> 95.9 us).
-  // (The dropout instances exist with 256-row blocks only.)
-  const int vec_scores =
-      aligned16(scores) && st[0] % 8 == 0 && st[1] % 8 == 0 && st[2] % 8 == 0 && pr.N % 8 == 0;
+  // One workgroup runs per CU, so with 256-row blocks in one round the
+  // longest row block sets the time.  Unpacked launches without dropout
+  // (whose instances have 256-row blocks only) then take 128- or 64-row
+  // blocks whose key tiles are split between wave pairs (KS2): half or a
+  // quarter of the rows, half the steps.  Measured (us, 256 / 128 / 64 rows):
+  //  * 64 rows while those blocks run in one round (B1 H12 S1000 D64 causal
+  //    33.5 / 20.9 / 18.2; B1 H32 S512 D128 full 24.4 / 17.6 / 16.2), and up
+  //    to 128-row blocks in one round for causal square problems with rows of
+  //    2048 keys or more, where two rounds of longest-first pairs balance
+  //    (B1 H8 S4096 131.9 / 93.1 / 82.6; B1 H12 M2048 N4096, not square:
+  //    132.5 / 80.2 / 101.5; unaligned rows, whose stores cost more, B1 H8
+  //    S4095: 173 / 142 / 170);
+  //  * 128 rows while those run in one round (B1 H32 S1024 full 41.2 / 31.4 /
+  //    43.0; B1 H12 S2000 D64 full 61.8 / 39.1 / 59.5);
+  //  * 128 rows in two rounds under a causal mask, whose mirror order balances
+  //    them, for rows of 1024 keys or more (B1 H16 S4096 164 / 131 / 182; B1
+  //    H32 S1280 50.2 / 37.5 / 51.8; B4 H32 S512 29.3 / 33.2 / 50.7), but when
+  //    they fill both rounds only for longer ones (B1 H32 S2048 90.4 / 96.7 /
+  //    111; B1 H16 S3072 103.8 / 78.4);
+  //  * else 256 rows (B1 H32 S2048 full 94.9 / 124.3 / 163.5; B2 H16 S1536 D64
+  //    full 45.1 / 53.7 / 60.7).
   const int64_t cus = device_cu_count();
-  if (pw.pack == 1 && !(a->dropout_p > 0.f) &&
-      (int64_t)pr.B * pr.H * ((pr.M + fas::kFwdRows - 1) / fas::kFwdRows) <= cus) {
-    bm = fas::kFwdRows / 2;
-    // When even the 128-row blocks all run in one round under a causal mask
-    // with long rows, the writer takes 64-row blocks with each block's key
-    // tiles split between its two wave pairs (16-byte score rows only): two
-    // rounds of balanced pairs.  A step of it moves twice the K/V bytes per
-    // score, so it pays only when the longest row block is long (measured:
-    // B1 H8 S4096 0.118 -> 0.096 ms; B1 H32 S1024 0.0367 -> 0.0383 ms).
-    if (vec_scores && pr.causal && pr.N >= 2048 &&
-        (int64_t)pr.B * pr.H * ((pr.M + bm - 1) / bm) <= cus)
-      bm = fas::kFwdRows / 4;
+  const int aligned = score_rows_aligned(scores, st, pr.N);
+  if (pw.pack == 1 && !(a->dropout_p > 0.f)) {
+    const int64_t heads = (int64_t)pr.B * pr.H;
+    const int64_t n256 = heads * ((pr.M + 255) / 256), n128 = heads * ((pr.M + 127) / 128),
+                  n64 = heads * ((pr.M + 63) / 64);
+    const bool square = pr.causal && pr.N - pr.M < pr.M / 4;
+    if (n64 <= cus || (n128 <= cus && square && pr.N >= 2048 && aligned))
+      bm = 64;
+    else if (n128 <= cus ||
+             (n256 <= cus && pr.causal && pr.N >= 1024 && (n128 <= cus * 7 / 4 || pr.N >= 3072)))
+      bm = 128;
   }
-  // 128-row blocks that all run in one round: the 8-wave key-split writer
-  // (two waves per SIMD on each block's even and odd key tiles).
-  const int key_split2 = bm == fas::kFwdRows / 2 && vec_scores &&
-                         (int64_t)pr.B * pr.H * ((pr.M + bm - 1) / bm) <= cus;
   fas::FwdParams p = fwd_params(a, pw, false, bm);
-  p.key_split2 = key_split2;
   rescale_dropout(p, a);
   p.scores = static_cast<uint16_t*>(scores);
   p.ss0 = st[0];
   p.ss1 = st[1];
   p.ss2 = st[2];
-  p.vec_scores = vec_scores;
+  p.scores_aligned = aligned;
   // The writer runs one workgroup per CU; with no more workgroups than CUs
   // they all run at once and each writes its own zero triangle.
   p.zero_self = (int64_t)p.nrb * (pr.B * pr.H / pw.pack) <= cus ? 1 : 0;

@@ -228,6 +228,31 @@ __device__ __forceinline__ void buf_store16_nt(u32x4 v, __amdgpu_buffer_rsrc_t r
   __builtin_amdgcn_raw_buffer_store_b128(v, r, off, soff, kAuxNT);
 }
 
+// Score stores.  ALN: every row starts on a 64-byte boundary, so a wave's
+// 128-byte row pieces are whole 64-byte halves of a line and stream past the
+// caches (kAuxNT).  Otherwise a row may start at any element: the pieces
+// share their first and last line with their neighbours', and the stores go
+// through the L2, which merges them (gfx950 runs in the unaligned access
+// mode: 16-byte stores at any 2-byte address).  Scores alone, B1 H32 S4096,
+// non-temporal against cached: N = 4096 204 / 300 us, N = 4128 (64-byte
+// rows) 249 / 397, N = 4112 (32-byte) 523 / 407, N = 4104 (16-byte) 682 /
+// 414; element-wise stores at N = 4095: 1527 us, now 305.
+template <bool ALN>
+__device__ __forceinline__ void store_score16(u32x4 v, __amdgpu_buffer_rsrc_t r, uint32_t off,
+                                              uint32_t soff = 0) {
+  __builtin_amdgcn_raw_buffer_store_b128(v, r, off, soff, ALN ? kAuxNT : 0);
+}
+// Elements 0 .. n-1 (n < 8) of v, one by one: the unit that the end of an
+// unaligned row cuts.
+__device__ __forceinline__ void store_score_tail(u32x4 v, __amdgpu_buffer_rsrc_t r, uint32_t off,
+                                                 uint32_t soff, int n) {
+#pragma unroll
+  for (int e = 0; e < 7; ++e)
+    if (e < n)
+      __builtin_amdgcn_raw_buffer_store_b16((uint16_t)(v[e >> 1] >> (16 * (e & 1))), r,
+                                            off + 2u * (uint32_t)e, soff, 0);
+}
+
 // a ^ b ^ c in one instruction (v_bitop3_b32; 0x96 is the truth table of the
 // three-way exclusive or over operand bytes 0xF0, 0xCC, 0xAA).
 __device__ __forceinline__ uint32_t xor3(uint32_t a, uint32_t b, uint32_t c) {

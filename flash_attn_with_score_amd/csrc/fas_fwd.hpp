@@ -38,8 +38,7 @@
 //    softmax (every term is divided by the same l at the end).
 //  * Masks are applied only on tiles that cross the causal diagonal or the
 //    key-length edge; all other tiles take an unmasked path.
-//  * Score writer (kFwdScores, 8 waves, or 4 with 128-row blocks when 256-row
-//    blocks would leave CUs idle): the first half of the waves ("loaders")
+//  * Score writer (kFwdScores): the first half of the waves ("loaders")
 //    fetch K/V and never store inside the loop, so their wait for the DMA is
 //    never a wait for stores; the second half ("storers") issue every global
 //    score store.
@@ -134,16 +133,19 @@ struct RowGeom {
 // one vector select and scalar bookkeeping.  The remaining blocks of each
 // run (fewer than eight, the last one possibly cut by N) are written by
 // tail() after the loop.
-template <bool PACK>
+// ROWCHK: rows past M are dropped by the lane's position (several packed
+// heads, or unaligned rows) instead of the buffer's extent.  ALN: see
+// store_score16; an unaligned row's last unit may be cut by N.
+template <bool ROWCHK, bool ALN>
 struct ZeroRuns {
   int run = 8;          // current run, 0-3 in a, 4-7 in b, 8 = no full batch left
   int nb = 0;           // full batches left in the current run
   uint32_t koff = 0;    // byte offset of the batch's first key
   uint32_t roff = 0;    // uniform offset of the current run's 8-row group
-  int lim = 0;          // PACK: positions of the current run's group below M
+  int lim = 0;          // ROWCHK: positions of the current run's group below M
   int ra = 0, rb = 0, za = 0, zb = 0, ca = 0, cb = 0, N = 0;
   uint32_t lane_off = 0;  // the lane's row in the group and its chunk
-  int lpos = 0;           // PACK: the lane's position within the group
+  int lpos = 0;           // ROWCHK: the lane's position within the group
   RowGeom geo;
 
   // 64-key blocks per row of a rectangle starting at key z whose first row
@@ -176,7 +178,7 @@ struct ZeroRuns {
   // voffset of store 0 of the current batch (kOffNone once no full batch is
   // left, or for a row past M); store i adds 128*i.
   __device__ __forceinline__ uint32_t vbase() const {
-    return run < 8 && (!PACK || lpos < lim) ? roff + lane_off : kOffNone;
+    return run < 8 && (!ROWCHK || lpos < lim) ? roff + lane_off : kOffNone;
   }
   __device__ __forceinline__ void advance() {
     koff += 1024u;
@@ -184,16 +186,19 @@ struct ZeroRuns {
       start(run == 3 && full_batches(N, cb) == 0 ? 8 : run + 1);
   }
   // Blocks of every run past its full batches, masked at key N.
-  template <class Store>
-  __device__ __forceinline__ void tail(int lane_key, Store&& store) const {
+  __device__ __forceinline__ void tail(int lane_key, __amdgpu_buffer_rsrc_t rz) const {
     for (int r = 0; r < 8; ++r) {
       const bool in_a = r < 4;
       const int c = in_a ? ca : cb, z = in_a ? za : zb;
       const uint32_t ro = geo.group_off(run_first(r));
-      const bool row_ok = !PACK || lpos < geo.M - (run_first(r) >> geo.shift);
+      const bool row_ok = !ROWCHK || lpos < geo.M - (run_first(r) >> geo.shift);
       for (int kb = 8 * full_batches(N, c); kb < c; ++kb) {
         const int k = z + 64 * kb;
-        store(lane_key < N - k && row_ok ? ro + lane_off : kOffNone, (uint32_t)k * 2u);
+        const int n = row_ok ? N - k - lane_key : 0;  // keys left from the lane's unit on
+        store_score16<ALN>(u32x4{0u, 0u, 0u, 0u}, rz, n >= (ALN ? 1 : 8) ? ro + lane_off : kOffNone,
+                           (uint32_t)k * 2u);
+        if (!ALN && n > 0 && n < 8)
+          store_score_tail(u32x4{0u, 0u, 0u, 0u}, rz, ro + lane_off, (uint32_t)k * 2u, n);
       }
     }
   }
@@ -243,8 +248,8 @@ __device__ __forceinline__ int64_t* region_rows() {
 // PACK: GQA packing (p.pack query heads per workgroup, per-lane heads and
 // positions); without it the workgroup's rows are one head's and every
 // per-lane head offset folds away at compile time.
-// Two waves per SIMD, except for the 4-wave score writer, whose LDS (one
-// workgroup per CU) allows one.
+// Two waves per SIMD, except for the 4-wave score writer (64-row blocks),
+// whose LDS (one workgroup per CU) allows one.
 // KS2 (unpacked score writer): row blocks of 32 * NW / 2 rows whose key
 // range is split between the wave pairs: loader wave i takes the even key
 // tiles and storer wave NW/2 + i the odd ones of the same 32 rows, so a step
@@ -254,17 +259,20 @@ __device__ __forceinline__ int64_t* region_rows() {
 // the kernel time:
 //  * 4 waves, 64-row blocks: two rounds whose longest-first pairs (rb,
 //    15 - rb) all take the same number of steps (one wave per SIMD);
-//  * 8 waves, 128-row blocks: one round at two waves per SIMD, half the steps
-//    of the 4-wave 128-row writer per row block.  Its K/V stages fill 128 KiB
+//  * 8 waves, 128-row blocks: two waves per SIMD, half the steps of the
+//    256-row writer per row block.  Its K/V stages fill 128 KiB
 //    of LDS, so the loaders' score tiles are single-buffered: a second
 //    barrier in each step (after the tiles are staged) hands them to the
 //    storers, which store both tiles of the step during O += P V.
-template <class E, int D, int MODE, int NW, bool DROP, bool PACK, bool KS2 = false>
+// ALN (score writer): whether the score rows start on 64-byte boundaries
+// (store_score16).
+template <class E, int D, int MODE, int NW, bool DROP, bool PACK, bool KS2 = false, bool ALN = true>
 __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(NW == 4 ? 1 : 2, 2)))
 void fwd_kernel(const FwdParams p) {
   static_assert(MODE != kFwdScores || NW == 8 || NW == 4, "the score writer uses 4 or 8 waves");
   static_assert(!KS2 || (MODE == kFwdScores && !DROP && !PACK),
                 "the key-split writer is the unpacked score writer");
+  static_assert(ALN || MODE == kFwdScores, "only the score writer has unaligned rows");
   constexpr int NH = NW / 2;  // score writer: loader waves [0, NH), storer waves [NH, NW)
   const int pack = PACK ? p.pack : 1;
   constexpr int KS = D / 16;               // MFMA k-steps over the head dim
@@ -432,17 +440,15 @@ void fwd_kernel(const FwdParams p) {
     }
   };
   // ---- score writer state (kFwdScores) ----
-  // Storers exist only for 16-byte aligned score rows; otherwise every wave
-  // writes its own scores element-wise.
-  const bool vec = MODE == kFwdScores && p.vec_scores != 0;
-  const bool storer = vec && !loader;
+  const bool storer = MODE == kFwdScores && !loader;
+  constexpr bool kRowChk = PACK || !ALN;  // rows past M are masked per lane
   const int pwave = wave - NH;  // the loader wave a storer serves
   const int pwtiles = kSplit ? wtiles_of(row0 + 32 * pwave) : 0;
   // Lane (row l/8, chunk l%8) of an 8-row x 128-byte store.
   int lane_key = 8 * (lane & 7);
   __amdgpu_buffer_rsrc_t rs = make_rsrc(p.scores, 0);
   __amdgpu_buffer_rsrc_t rz = rs;
-  ZeroRuns<PACK> zr;
+  ZeroRuns<kRowChk, ALN> zr;
   // Score rows (RowGeom): the storer's stores address rows 8i + l/8 of a
   // 32-row wave tile through the lane's fixed offset plus a uniform part.
   const int sshift = PACK ? p.pack_shift : 0;
@@ -457,8 +463,12 @@ void fwd_kernel(const FwdParams p) {
     const uint32_t hspan = (uint32_t)((pack - 1) * p.ss1 * 2);
     const int pos0 = min(p.M, pos_lo(row0));
     const int pos1 = min(p.M, pos_lo(row0 + BM - 1) + 1);
-    rs = make_rsrc(p.scores + b * p.ss0 + h0 * p.ss1 + (int64_t)pos0 * p.ss2,
-                   __builtin_amdgcn_readfirstlane(hspan + (uint32_t)((pos1 - pos0) * p.ss2 * 2)));
+    auto extent = [&](int n) {  // bytes of n rows (unaligned rows may be closer than N: n = 1)
+      return __builtin_amdgcn_readfirstlane(
+          hspan + (ALN ? (uint32_t)(n * p.ss2 * 2)
+                       : n > 0 ? (uint32_t)(((n - 1) * p.ss2 + p.N) * 2) : 0u));
+    };
+    rs = make_rsrc(p.scores + b * p.ss0 + h0 * p.ss1 + (int64_t)pos0 * p.ss2, extent(pos1 - pos0));
     gs = RowGeom{sshift, p.M, pos0, (uint32_t)(p.ss2 * 2), (uint32_t)(p.ss1 * 2)};
     lane_off = gs.lane_off(lane);
     // Zeros of the mirror row block, or of its own when every workgroup
@@ -468,7 +478,7 @@ void fwd_kernel(const FwdParams p) {
     const int mpos0 = min(p.M, pos_lo(mrow0));
     const int mpos1 = min(p.M, pos_lo(mrow0 + BM - 1) + 1);
     rz = make_rsrc(p.scores + b * p.ss0 + h0 * p.ss1 + (int64_t)mpos0 * p.ss2,
-                   __builtin_amdgcn_readfirstlane(hspan + (uint32_t)((mpos1 - mpos0) * p.ss2 * 2)));
+                   extent(mpos1 - mpos0));
     if (storer) {
       RowGeom gz = gs;
       gz.pos0 = mpos0;
@@ -514,12 +524,29 @@ void fwd_kernel(const FwdParams p) {
   // Rows 8i + l/8 of the wave tile starting at virtual row T, keys k0..
   auto staged_offsets = [&](int T, int k0, bool valid, uint32_t (&o)[4])
                             __attribute__((always_inline)) {
-    const bool ok = valid && k0 + lane_key < p.N;
+    const bool ok = valid && k0 + lane_key + (ALN ? 0 : 7) < p.N;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const int V = T + 8 * i;
-      const bool row_ok = !PACK || lpos < p.M - (V >> sshift);
+      const bool row_ok = !kRowChk || lpos < p.M - (V >> sshift);
       o[i] = ok && row_ok ? gs.group_off(V) + (uint32_t)(k0 * 2) + lane_off : kOffNone;
+    }
+  };
+  // Unaligned rows: the 16-byte unit that key N cuts (keys N & ~7 .. N - 1,
+  // in the last key tile) leaves element by element from the wave that
+  // computed it.
+  auto row_end = [&](const f32x16 (&s)[2], int k0) __attribute__((always_inline)) {
+    if constexpr (!ALN) {
+      if (k0 + BN <= p.N || !row_ok) return;
+      uint16_t* sr = p.scores + b * p.ss0 + qh * p.ss1 + (int64_t)qpos * p.ss2;
+#pragma unroll
+      for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          const int key = k0 + 32 * kb + acc_row(r, g);
+          const float x = s[kb][r];
+          if (key >= (p.N & ~7) && key < p.N) sr[key] = E::cvt(x == neg_inf() ? 0.f : x * p.sm_scale);
+        }
     }
   };
   // One batch of kZero = 8 zero stores.
@@ -527,7 +554,7 @@ void fwd_kernel(const FwdParams p) {
     const uint32_t vb = zr.vbase();
 #pragma unroll
     for (int i = 0; i < kZero; ++i)
-      buf_store16_nt(u32x4{0u, 0u, 0u, 0u}, rz, vb + 128u * (uint32_t)i, zr.koff);
+      store_score16<ALN>(u32x4{0u, 0u, 0u, 0u}, rz, vb + 128u * (uint32_t)i, zr.koff);
     zr.advance();
   };
   // Score tiles of step t of the partner (staged by wave pwave in step t)
@@ -799,14 +826,14 @@ void fwd_kernel(const FwdParams p) {
             score_tile(kt, s, tw, std::true_type{});
             if constexpr (!NZ) {
 #pragma unroll
-              for (int i = 0; i < 8; ++i) buf_store16_nt(w[i], rs, o[i]);
+              for (int i = 0; i < 8; ++i) store_score16<ALN>(w[i], rs, o[i]);
               sched_score_tile<KS, 8>();
             } else {
               sched_score_tile<KS, 0>();
             }
           } else {
 #pragma unroll
-            for (int i = 0; i < 8; ++i) buf_store16_nt(w[i], rs, o[i]);
+            for (int i = 0; i < 8; ++i) store_score16<ALN>(w[i], rs, o[i]);
           }
         } else if (act) {
           score_tile(kt, s, tw, std::true_type{});
@@ -816,6 +843,7 @@ void fwd_kernel(const FwdParams p) {
         if (act) {
           if (masked) apply_mask(s, k0);
           stage_tile((loader ? wave : kOwnStg + pwave) * TSZ, s, masked);
+          if (masked) row_end(s, k0);
           update_offset_of(s);
           u32x4 pb[4];
           l_i += make_p(s, pb);
@@ -828,7 +856,7 @@ void fwd_kernel(const FwdParams p) {
           if constexpr (ST) {
             if constexpr (NZ) {
 #pragma unroll
-              for (int i = 0; i < 8; ++i) buf_store16_nt(w[i], rs, o[i]);
+              for (int i = 0; i < 8; ++i) store_score16<ALN>(w[i], rs, o[i]);
             } else {
               zero_batch();
             }
@@ -848,7 +876,7 @@ void fwd_kernel(const FwdParams p) {
           score_tile(kt, s, tw, std::integral_constant<bool, kSplit>{});
           if constexpr (!NZ) {
 #pragma unroll
-            for (int i = 0; i < 8; ++i) buf_store16_nt(w[i], rs, o[i]);
+            for (int i = 0; i < 8; ++i) store_score16<ALN>(w[i], rs, o[i]);
             sched_score_tile<KS, 8>();
           } else {
             sched_score_tile<KS, 0>();
@@ -860,31 +888,20 @@ void fwd_kernel(const FwdParams p) {
         if (masked) apply_mask(s, k0);
 
         if constexpr (MODE == kFwdScores) {
-          if (vec) {
-            if (loader) {
-              stage_tile((stage * NH + wave) * TSZ, s, masked);
-            } else {
-              // The storer reads this tile back row-major in the next key
-              // tile (staged_pair), from other lanes of the same wave.  A
-              // wave's LDS accesses execute in issue order, so only the
-              // compiler must keep the order: the wave barrier keeps this
-              // iteration's read-back before these writes, and the step's
-              // closing lds_barrier (an asm with a memory clobber) keeps the
-              // writes before the next iteration's read-back.
-              __builtin_amdgcn_wave_barrier();
-              stage_tile((NW + pwave) * TSZ, s, masked);
-            }
-          } else if (row_ok) {
-            uint16_t* sr = p.scores + b * p.ss0 + qh * p.ss1 + (int64_t)qpos * p.ss2;
-#pragma unroll
-            for (int kb = 0; kb < 2; ++kb)
-#pragma unroll
-              for (int r = 0; r < 16; ++r) {
-                const int key = k0 + 32 * kb + acc_row(r, g);
-                const float x = s[kb][r];
-                if (key < p.N) sr[key] = E::cvt(x == neg_inf() ? 0.f : x * p.sm_scale);
-              }
+          if (loader) {
+            stage_tile((stage * NH + wave) * TSZ, s, masked);
+          } else {
+            // The storer reads this tile back row-major in the next key
+            // tile (staged_pair), from other lanes of the same wave.  A
+            // wave's LDS accesses execute in issue order, so only the
+            // compiler must keep the order: the wave barrier keeps this
+            // iteration's read-back before these writes, and the step's
+            // closing lds_barrier (an asm with a memory clobber) keeps the
+            // writes before the next iteration's read-back.
+            __builtin_amdgcn_wave_barrier();
+            stage_tile((NW + pwave) * TSZ, s, masked);
           }
+          if (masked) row_end(s, k0);
         }
         if constexpr (MODE == kFwdRowSum) {
           // Masked scores (-inf) count as 0; only the masked loop copy can
@@ -1015,7 +1032,7 @@ void fwd_kernel(const FwdParams p) {
           pv_mma(pb, vt);
           if constexpr (NZ) {
 #pragma unroll
-            for (int i = 0; i < 8; ++i) buf_store16_nt(w[i], rs, o[i]);
+            for (int i = 0; i < 8; ++i) store_score16<ALN>(w[i], rs, o[i]);
           } else {
             zero_batch();
           }
@@ -1028,7 +1045,7 @@ void fwd_kernel(const FwdParams p) {
         uint32_t o[8];
         staged_pair(it - 1, w, o);
 #pragma unroll
-        for (int i = 0; i < 8; ++i) buf_store16_nt(w[i], rs, o[i]);
+        for (int i = 0; i < 8; ++i) store_score16<ALN>(w[i], rs, o[i]);
         zero_batch();
       }
       if (loader) vm_wait_all();
@@ -1085,20 +1102,9 @@ void fwd_kernel(const FwdParams p) {
       uint32_t o[8];
       staged_pair(t_end - 1, w, o);
 #pragma unroll
-      for (int i = 0; i < 8; ++i) buf_store16_nt(w[i], rs, o[i]);
+      for (int i = 0; i < 8; ++i) store_score16<ALN>(w[i], rs, o[i]);
       while (zr.pending()) zero_batch();
-      zr.tail(lane_key, [&](uint32_t vo, uint32_t so) {
-        buf_store16_nt(u32x4{0u, 0u, 0u, 0u}, rz, vo, so);
-      });
-    }
-    if (!vec) {  // element-wise zero triangle for unaligned rows
-      const int z0 = min(p.N, wtiles * BN);
-      for (int rr = 0; rr < 32; ++rr) {
-        const int v = wrow0 + rr, pos = v / pack;
-        if (pos >= p.M) break;
-        uint16_t* sr = p.scores + b * p.ss0 + (h0 + v - pos * pack) * p.ss1 + (int64_t)pos * p.ss2;
-        for (int key = z0 + lane; key < p.N; key += 64) sr[key] = 0;
-      }
+      zr.tail(lane_key, rz);
     }
   }
 
@@ -1251,12 +1257,12 @@ __global__ __launch_bounds__(256) void fwd_combine_kernel(const FwdParams p) {
   }
 }
 
-template <class E, int D, int MODE, int NW, bool DROP, bool PACK, bool KS2 = false>
+template <class E, int D, int MODE, int NW, bool DROP, bool PACK, bool KS2 = false, bool ALN = true>
 hipError_t launch_fwd_t(const FwdParams& p, hipStream_t stream) {
   constexpr bool kCanSplit = MODE == kFwdPlain || MODE == kFwdPlainKeepBits || MODE == kFwdRowSum;
   const int64_t nsplit = kCanSplit ? p.nsplit : 1;
   const dim3 grid((unsigned)((int64_t)p.nrb * (p.B * p.H / p.pack) * nsplit)), block(NW * 64);
-  hipLaunchKernelGGL((fwd_kernel<E, D, MODE, NW, DROP, PACK, KS2>), grid, block, 0, stream, p);
+  hipLaunchKernelGGL((fwd_kernel<E, D, MODE, NW, DROP, PACK, KS2, ALN>), grid, block, 0, stream, p);
   if constexpr (kCanSplit) {
     if (p.nsplit > 1 && p.M > 0) {
       const int64_t nblk = (p.M + 2048 / D - 1) / (2048 / D);
@@ -1268,21 +1274,22 @@ hipError_t launch_fwd_t(const FwdParams& p, hipStream_t stream) {
   return hipGetLastError();
 }
 
-template <int MODE, int NW, bool DROP = false, bool PACK = false, bool KS2 = false>
+template <int MODE, int NW, bool DROP = false, bool PACK = false, bool KS2 = false,
+          bool ALN = true>
 hipError_t launch_fwd_mode(const FwdParams& p, int dtype, int d, hipStream_t s) {
   if (dtype == 0) {
     switch (d) {
-      case 16: return launch_fwd_t<F16, 16, MODE, NW, DROP, PACK, KS2>(p, s);
-      case 32: return launch_fwd_t<F16, 32, MODE, NW, DROP, PACK, KS2>(p, s);
-      case 64: return launch_fwd_t<F16, 64, MODE, NW, DROP, PACK, KS2>(p, s);
-      case 128: return launch_fwd_t<F16, 128, MODE, NW, DROP, PACK, KS2>(p, s);
+      case 16: return launch_fwd_t<F16, 16, MODE, NW, DROP, PACK, KS2, ALN>(p, s);
+      case 32: return launch_fwd_t<F16, 32, MODE, NW, DROP, PACK, KS2, ALN>(p, s);
+      case 64: return launch_fwd_t<F16, 64, MODE, NW, DROP, PACK, KS2, ALN>(p, s);
+      case 128: return launch_fwd_t<F16, 128, MODE, NW, DROP, PACK, KS2, ALN>(p, s);
     }
   } else {
     switch (d) {
-      case 16: return launch_fwd_t<BF16, 16, MODE, NW, DROP, PACK, KS2>(p, s);
-      case 32: return launch_fwd_t<BF16, 32, MODE, NW, DROP, PACK, KS2>(p, s);
-      case 64: return launch_fwd_t<BF16, 64, MODE, NW, DROP, PACK, KS2>(p, s);
-      case 128: return launch_fwd_t<BF16, 128, MODE, NW, DROP, PACK, KS2>(p, s);
+      case 16: return launch_fwd_t<BF16, 16, MODE, NW, DROP, PACK, KS2, ALN>(p, s);
+      case 32: return launch_fwd_t<BF16, 32, MODE, NW, DROP, PACK, KS2, ALN>(p, s);
+      case 64: return launch_fwd_t<BF16, 64, MODE, NW, DROP, PACK, KS2, ALN>(p, s);
+      case 128: return launch_fwd_t<BF16, 128, MODE, NW, DROP, PACK, KS2, ALN>(p, s);
     }
   }
   return hipErrorInvalidValue;

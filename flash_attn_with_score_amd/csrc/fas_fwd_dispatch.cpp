@@ -6,6 +6,7 @@ namespace fas {
 hipError_t launch_fwd_plain(const FwdParams& p, int dtype, int d, hipStream_t s);
 hipError_t launch_fwd_rowsum(const FwdParams& p, int dtype, int d, hipStream_t s);
 hipError_t launch_fwd_scores(const FwdParams& p, int dtype, int d, hipStream_t s);
+hipError_t launch_fwd_scores_unaligned(const FwdParams& p, int dtype, int d, hipStream_t s);
 hipError_t launch_fwd_region(const FwdParams& p, int dtype, int d, hipStream_t s);
 hipError_t launch_fwd_dropout(const FwdParams& p, int mode, int dtype, int d, hipStream_t s);
 hipError_t launch_fwd_packed(const FwdParams& p, int mode, int dtype, int d, hipStream_t s);
@@ -14,14 +15,15 @@ hipError_t launch_fwd_scores_packed(const FwdParams& p, int dtype, int d, hipStr
 // GQA-packed launches (p.pack > 1) take their own instances; the host never
 // packs a launch with dropout.
 hipError_t launch_fwd(const FwdParams& p, int mode, int dtype, int d, hipStream_t s) {
-  // Only the unpacked score writer without dropout has 128-row and (key
-  // split, 16-byte score rows) 64-row instances; every other launch is built
-  // for 256-row blocks.
+  // Only the unpacked score writer without dropout has 128- and 64-row
+  // instances; every other launch is built for 256-row blocks.
   const bool small_writer = mode == kFwdScores && p.pack == 1 && !p.dropout &&
-                            ((p.bm == kFwdRows / 2 && (!p.key_split2 || p.vec_scores)) ||
-                             (p.bm == kFwdRows / 4 && p.vec_scores));
-  if (p.key_split2 && !(small_writer && p.bm == kFwdRows / 2)) return hipErrorInvalidValue;
+                            (p.bm == kFwdRows / 2 || p.bm == kFwdRows / 4);
   if (p.bm != kFwdRows && !small_writer) return hipErrorInvalidValue;
+  if (mode == kFwdScores && !p.scores_aligned) {
+    if (p.pack > 1 && p.dropout) return hipErrorInvalidValue;
+    return launch_fwd_scores_unaligned(p, dtype, d, s);
+  }
   if (p.pack > 1) {
     if (p.dropout && mode != kFwdRegion) return hipErrorInvalidValue;
     return mode == kFwdScores ? launch_fwd_scores_packed(p, dtype, d, s)

@@ -80,13 +80,11 @@ struct FwdParams {
   int pack;
   int pack_shift;    // log2(pack) when pack is 1, 2, 4 or 8 (the score writer's packings)
   int nrb;           // virtual row blocks per group of `pack` heads
-  int bm;            // rows per workgroup (32 per wave; the score writer takes 128 or 256)
-  int vec_scores;    // scores rows 16-byte aligned and N % 8 == 0
+  int bm;            // rows per workgroup (256, the score writer also 128 or 64)
+  int scores_aligned;  // score rows start on 64-byte boundaries and N % 8 == 0
   int zero_self;     // score writer: 1 = a workgroup writes its own row block's zeros
                      // (all workgroups run at once), 0 = its mirror row block's
   int vec_region;    // split % 8 == 0
-  int key_split2;    // score writer with 128-row blocks: 1 = the 8-wave key-split
-                     // instance (wave pairs take the even and odd key tiles)
   int dropout;       // 1: the dropout instances (modes other than kFwdRegion)
   DropParams drop;   // scale also applies in the key-split combine (1 without dropout)
   // kFwdPlainKeepBits: the keep decisions as bits, word
@@ -282,7 +280,7 @@ struct ScoresParams {
   // head (pshift > 0 only under GQA, 2^pshift * M <= 512), its virtual rows
   // v = m * 2^pshift + j holding position m of head h0 + j.
   int pshift;
-  int vec;            // base and row strides 16-byte aligned, N % 8 == 0: 16-byte stores
+  int aligned;        // score rows start on 64-byte boundaries and N % 8 == 0
   float sm_scale;     // signed
 };
 

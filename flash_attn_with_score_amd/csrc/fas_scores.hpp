@@ -65,12 +65,12 @@ __device__ __forceinline__ void scores_load_keys(u32x4 (&a0)[D / 16], u32x4 (&a1
 // One wave's 32 x 64 score tile: query rows wrow0 + c (their Q rows at row
 // qrow + c of the LDS tile qt) against keys [k0, k0 + 64) held in a0 / a1,
 // scaled by sm_scale, masked, converted and stored through the wave's LDS
-// stage st.  VEC_ONLY: the caller runs only with p.vec set (no per-element
-// store path).
+// stage st.  ALN: score rows on 64-byte boundaries (store_score16); otherwise
+// the 16-byte unit that key N cuts leaves element by element.
 // GROUP (the resident-Q kernel): rows are the virtual rows of a head group
 // (2^p.pshift heads from shead on) and every lane's store carries its own
 // validity, past M or N at kOffNoneScores.
-template <class E, int D, bool MASK, bool VEC_ONLY = false, bool GROUP = false>
+template <class E, int D, bool MASK, bool ALN, bool GROUP = false>
 __device__ __forceinline__ void scores_tile(const ScoresParams& p, const uint16_t* qt, int qrow,
                                             const u32x4 (&a0)[D / 16], const u32x4 (&a1)[D / 16],
                                             u32x4* st, uint16_t* shead, int wrow0, int k0,
@@ -97,10 +97,13 @@ __device__ __forceinline__ void scores_tile(const ScoresParams& p, const uint16_
       s[1] = E::mma(a1[ks], qb[ks], s[1]);
     }
   }
-  const bool key_ok = k0 + 8 * (lane & 7) < p.N;  // the lane's store unit lies below N
+  // The lane's store unit lies below N; its elements below N where N cuts it.
+  const int key_n = p.N - (k0 + 8 * (lane & 7));
+  const bool key_ok = key_n >= (ALN ? 1 : 8);
+  const bool row_end = !ALN && k0 + 64 > p.N;  // wave-uniform
   // The lane's query row (its position within the head for a group).
   const int row = GROUP ? (wrow0 + c) >> p.pshift : wrow0 + c;
-  if (VEC_ONLY || p.vec) {
+  {
     // Stage row c, 16-byte unit u = 4j + 2hf + g at c*8 + (u ^ ((c/2) & 7)):
     // conflict-free for these writes (one unit of 32 rows) and for the
     // row-major reads below (8 units of 8 rows).  The stage is private to
@@ -138,10 +141,12 @@ __device__ __forceinline__ void scores_tile(const ScoresParams& p, const uint16_
       for (int i = 0; i < 4; ++i) {
         const int r = (lane >> 3) + 8 * i, mr = r >> p.pshift;
         const u32x4 val = st[r * 8 + (u ^ ((r >> 1) & 7))];
-        buf_store16_nt(val, rs,
-                       key_ok && m0 + mr < p.M
-                           ? (uint32_t)(((r & jm) * p.ss1 + mr * p.ss2 + 8 * u) * 2)
-                           : kOffNoneScores);
+        const uint32_t off = m0 + mr < p.M
+                                 ? (uint32_t)(((r & jm) * p.ss1 + mr * p.ss2 + 8 * u) * 2)
+                                 : kOffNoneScores;
+        store_score16<ALN>(val, rs, key_ok ? off : kOffNoneScores);
+        if (row_end && key_n > 0 && key_n < 8 && off != kOffNoneScores)
+          store_score_tail(val, rs, off, 0, key_n);
       }
     } else {
       // The buffer ends at the wave's last key below N in its last row below
@@ -157,31 +162,22 @@ __device__ __forceinline__ void scores_tile(const ScoresParams& p, const uint16_
       for (int i = 0; i < 4; ++i) {
         const int r = (lane >> 3) + 8 * i;
         const u32x4 val = st[r * 8 + (u ^ ((r >> 1) & 7))];
-        buf_store16_nt(val, rs, key_ok ? (uint32_t)((r * p.ss2 + 8 * u) * 2) : kOffNoneScores);
+        // (Unaligned rows may be closer than N: M = 1 with any row stride.)
+        const bool row_ok = ALN || r < nrows;
+        const uint32_t off = row_ok ? (uint32_t)((r * p.ss2 + 8 * u) * 2) : kOffNoneScores;
+        store_score16<ALN>(val, rs, key_ok ? off : kOffNoneScores);
+        if (row_end && key_n > 0 && key_n < 8 && row_ok) store_score_tail(val, rs, off, 0, key_n);
       }
     }
-  } else if (!VEC_ONLY && row < p.M) {
-    uint16_t* sr = shead + (int64_t)row * p.ss2;
-#pragma unroll
-    for (int j = 0; j < 2; ++j)
-#pragma unroll
-      for (int hf = 0; hf < 2; ++hf)
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          const int key = k0 + 32 * j + 16 * hf + 8 * g + e;
-          float v = s[j][8 * hf + e] * p.sm_scale;
-          if (MASK && p.causal_off + row < key) v = 0.f;
-          if (key < p.N) sr[key] = E::cvt(v);
-        }
   }
 }
 
 // MASK: the causal / key-range mask of attention_with_scores (entries with
 // key > causal_off + row written as 0); a template flag, so the unmasked
-// instance (compute_attention_scores) carries no per-score compare.  VEC:
-// p.vec is set (every step issues the same four stores per lane, so the
-// wait for the next step's Q leaves the step's stores in flight).
-template <class E, int D, bool MASK, bool VEC>
+// instance (compute_attention_scores) carries no per-score compare.  ALN:
+// p.aligned is set.  Every step issues the same four stores per lane, so the
+// wait for the next step's Q leaves the step's stores in flight.
+template <class E, int D, bool MASK, bool ALN>
 __global__ __launch_bounds__(64 * kScoresWaves) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void scores_kernel(const ScoresParams p) {
   constexpr int KS = D / 16;
@@ -261,7 +257,7 @@ void scores_kernel(const ScoresParams p) {
     if (t + 1 < t_end) load_q(t + 1);
     const int row0 = t * kScoresRows;      // the step's first row
     const int wrow0 = row0 + 32 * rg;      // the wave's first row
-    scores_tile<E, D, MASK, VEC>(p, qtile[stage], 32 * rg, a0, a1, st, shead, wrow0, k0, lane);
+    scores_tile<E, D, MASK, ALN>(p, qtile[stage], 32 * rg, a0, a1, st, shead, wrow0, k0, lane);
     if (t + 1 < t_end) write_q(stage ^ 1);
     lds_barrier();
   }
@@ -284,8 +280,8 @@ void scores_kernel(const ScoresParams p) {
 // of 256-key blocks: 97 against 52 us at B1 H32 N32768), and each step
 // writes 1 KiB runs of 32 rows.  With up to 160 KiB of LDS (D = 128, 512
 // rows) and up to 256 VGPRs one workgroup (8 waves, two per SIMD) runs per
-// CU.  Whole 16-byte score stores only (p.vec).
-template <class E, int D, bool MASK, int ROWS>
+// CU.
+template <class E, int D, bool MASK, int ROWS, bool ALN>
 __global__ __launch_bounds__(64 * kScoresWaves) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void scores_qres_kernel(const ScoresParams p) {
   static_assert(ROWS == 32 || ROWS == 64 || ROWS == 128 || ROWS == 256 || ROWS == 512,
@@ -368,7 +364,7 @@ void scores_qres_kernel(const ScoresParams p) {
     // 256-VGPR budget).
 #pragma unroll 8
     for (int t = 0; t < NST; ++t)
-      scores_tile<E, D, MASK, true, true>(p, qtile + 32 * D * t, 0, x0, x1, st, shead, 32 * t, k0,
+      scores_tile<E, D, MASK, ALN, true>(p, qtile + 32 * D * t, 0, x0, x1, st, shead, 32 * t, k0,
                                           lane);
   };
   auto load = [&](u32x4(&x0)[KS], u32x4(&x1)[KS], int kb) __attribute__((always_inline)) {

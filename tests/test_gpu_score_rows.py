@@ -1,0 +1,76 @@
+"""Score rows that do not start on 64-byte boundaries.
+
+Each case writes the scores through the C ABI into the middle of a buffer
+filled with a sentinel, with a row pitch of its own: every score must match
+the oracle, and the gaps between rows and the space around the matrix must
+keep the sentinel.  The shapes take each writer: key-split 64- and 128-row
+blocks, 256-row blocks, packed query heads, dropout, and the scores-only
+kernels (few and many query rows, behind the key-split forward).
+"""
+from __future__ import annotations
+
+import ctypes
+
+import pytest
+import torch
+
+from flash_attn_with_score_amd import _native
+from oracle import inputs, naive
+from tests.tolerances import assert_out_close, assert_scores_close
+
+pytestmark = pytest.mark.gpu
+
+SENTINEL = 0x5A5A
+# (B, Hq, Hk, M, N, D, causal, pitch - N, first element)
+CASES = [
+    (1, 4, 4, 130, 77, 64, True, 0, 0),       # 64-row blocks, N % 8 = 5
+    (1, 4, 4, 65, 201, 128, False, 3, 1),     # odd pitch, odd first element
+    (1, 2, 2, 64, 64, 32, True, 1, 0),        # whole tile, unaligned pitch
+    (1, 3, 3, 70, 72, 16, False, 0, 8),       # 16-byte rows
+    (1, 3, 3, 70, 96, 64, True, 0, 32),       # 64-byte rows
+    (1, 3, 3, 70, 90, 64, True, 6, 32),       # 64-byte rows, N % 8 = 2
+    (1, 130, 130, 100, 75, 16, False, 0, 0),  # 128-row blocks, one round
+    (1, 64, 64, 520, 1031, 16, True, 0, 3),   # 128-row blocks, two rounds
+    (1, 300, 300, 33, 67, 16, False, 0, 0),   # 256-row blocks
+    (1, 300, 300, 70, 70, 32, True, 2, 5),    # 256-row blocks, causal zeros
+    (1, 8, 2, 90, 131, 64, True, 0, 0),       # four packed heads
+    (1, 7, 1, 66, 129, 64, True, 4, 2),       # seven heads, unpacked writer
+    (1, 2, 2, 1, 7, 64, True, 0, 1),          # less than one 16-byte unit
+    (1, 2, 2, 7, 2049, 64, True, 0, 0),       # key split, resident-Q scores
+    (2, 4, 2, 3, 4100, 128, True, 1, 0),      # the same over two packed heads
+    (1, 2, 2, 700, 3001, 32, True, 0, 0),     # key split, K-resident scores
+]
+
+
+@pytest.mark.parametrize("case", CASES, ids=lambda c: "B{}H{}K{}M{}N{}D{}{}p{}o{}".format(*c))
+@pytest.mark.parametrize("dropout", [0.0, 0.2])
+def test_unaligned_score_rows(case, dropout, gpu):
+    B, Hq, Hk, M, N, D, causal, gap, first = case
+    print(f"[case] score rows {case} dropout={dropout}", flush=True)
+    lib = _native.load()
+    q, k, v = inputs.make_qkv(B, Hq, Hk, M, N, D, dtype=torch.float16, seed=5)
+    qd, kd, vd = q.to(gpu), k.to(gpu), v.to(gpu)
+    o = torch.full_like(qd, float("nan"))
+    drop = (dropout, 11, 4) if dropout else None
+    args = _native.make_args(qd, kd, vd, o, causal, D ** -0.5, drop)
+    nbytes = lib.fas_workspace_bytes(_native.VARIANT_SCORES, ctypes.byref(args), 0)
+    ws = torch.empty(nbytes + 256, dtype=torch.uint8, device=gpu)
+    wptr = ws.data_ptr() + (-ws.data_ptr()) % 256
+    pitch, lead = N + gap, 128 + first
+    rows = B * Hq * M
+    buf = torch.full((lead + rows * pitch + 256,), SENTINEL, dtype=torch.int16, device=gpu)
+    st = _native._I64x4(Hq * M * pitch, M * pitch, pitch, 1)
+    rc = lib.fas_attention_with_scores(ctypes.byref(args), buf.data_ptr() + 2 * lead, st, wptr,
+                                       nbytes, torch.cuda.current_stream().cuda_stream)
+    _native.check(lib, rc, "fas_attention_with_scores")
+    torch.cuda.synchronize()
+    body = buf[lead:lead + rows * pitch].view(rows, pitch)
+    assert (buf[:lead] == SENTINEL).all() and (buf[lead + rows * pitch:] == SENTINEL).all()
+    assert (body[:, N:] == SENTINEL).all()
+    got = body[:, :N].contiguous().view(torch.float16).view(B, Hq, M, N)
+    heads = sorted({0, 1, Hq // 2, Hq - 1})
+    ref = naive.reference_forward(q, k, v, causal=causal, want=("out", "scores"), heads=heads)
+    assert_scores_close(got[:, heads], ref["scores"][:, heads])
+    assert torch.isfinite(got.float()).all()
+    if not dropout:
+        assert_out_close(o[:, heads], ref["out"][:, heads])
