@@ -765,7 +765,9 @@ int run_softmax(const char* fn, int variant, const fas_attn_args* a, int64_t spl
   c.region_rows = p.region_rows;
   c.sq0 = p.sq0; c.sq1 = p.sq1; c.sq2 = p.sq2;
   c.sk0 = p.sk0; c.sk1 = p.sk1; c.sk2 = p.sk2;
-  c.q_bytes = p.q_bytes;
+  // One head's rows (p.q_bytes spans a packed group): steps past M read zeros,
+  // not the rows of the next head or the memory behind q.
+  c.q_bytes = slice_bytes(pr.M, p.sq2, pr.D);
   c.k_bytes = p.k_bytes;
   c.qneg = p.qneg;
   c.B = pr.B; c.H = pr.H; c.G = pr.G; c.M = pr.M; c.N = pr.N;

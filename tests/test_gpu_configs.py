@@ -196,3 +196,20 @@ def test_softmax_sums_head_split_plans(case, gpu):
     # Repeat calls: the same bits (the fold adds partials in split order).
     _, col2 = fas.attention_with_softmax_col_sum(qd, kd, vd, causal=True)
     assert torch.equal(col, col2)
+
+
+@pytest.mark.parametrize("M", [1, 100, 130])
+def test_softmax_col_sum_reads_no_row_past_q(M, gpu):
+    """Grouped query heads: q is the front part of a buffer whose rest is NaN,
+    and the column pass's last, partial step of 128 rows must not take rows
+    from behind the last head (they would turn every column into NaN)."""
+    B, Hq, Hk, N, D = 1, 8, 2, 300, 64
+    print(f"[case] col softmax, NaN behind q, M {M}", flush=True)
+    q, k, v = inputs.make_qkv(B, Hq, Hk, M, N, D, dtype=torch.float16, seed=3)
+    buf = torch.full((4 * Hq, M + 128, D), float("nan"), dtype=torch.float16, device=gpu)
+    qd = buf.view(-1)[:Hq * M * D].view(B, Hq, M, D)
+    qd.copy_(q)
+    _, col = fas.attention_with_softmax_col_sum(qd, k.to(gpu), v.to(gpu), causal=False)
+    torch.cuda.synchronize()
+    ref = naive.reference_forward(q, k, v, causal=False, want=("col_softmax",))
+    assert_sum_close(col, ref["col_softmax"], "col_softmax")
