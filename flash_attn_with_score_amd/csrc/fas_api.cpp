@@ -324,7 +324,7 @@ int zero_out3(const char* fn, float* out, const int64_t* st, int64_t n0, int64_t
 size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 
 struct SplitPlan {
-  int nsplit = 1, tps = 0;
+  int nsplit = 1;  // most workgroups per row block (the launch may take fewer)
   int64_t mpad = 0;
 };
 
@@ -387,20 +387,26 @@ struct Workspace {
 // Key split of the plain / row-sum forward.  When the row blocks of the
 // whole problem give fewer workgroups than the chip has CUs (short query
 // ranges against long key ranges: decode, last-window scoring), each row
-// block's key tiles are dealt to nsplit workgroups of at least 8 tiles,
-// aiming at ~512 workgroups in all.  Depends on sizes only, so the workspace
-// query and the launch agree.  The scores variant writes its scores in a second kernel on this
+// block's key tiles may be dealt to several workgroups of at least 8 tiles
+// (2 for at most 32 query rows per KV head, whose partials are small), up to
+// ~512 workgroups in all.  Depends on sizes only, so the workspace query and
+// the launch agree; fwd_plan picks the number of splits within it.
+// The scores variant writes its scores in a second kernel on this
 // route, so it splits only where the fused writer keeps few CUs busy for
-// long: up to 32 row blocks from 2048 keys on when the key range is at least
-// twice the query range (us, split against fused, B1 D128 causal: H4 M2048
-// N4096 57 / 67; H1 M1024 N2048 41 / 37; H12 M1024 N1024 44 / 24; H4 M256
-// N1024 36 / 23), up to 128 at 8 times (B2 H32 M512 N16384 607 / 734; H12
+// long: from 2048 keys on (us, split against fused, B1 D128 causal: H4 M64
+// N1024 24 / 22; H4 M256 N1024 36 / 23; H12 M1024 N1024 44 / 24), up to 32
+// row blocks over 4096 keys when the key range is at least twice the query
+// range (H4 M2048 N4096 57 / 67; H1 M1024 N2048 41 / 37), up to 128 at 8
+// times (B2 H32 M512 N16384 607 / 734; H12
 // M1024 N4096 96 / 68), and up to 256 at 64 times (B8 H32 M256 N16384 1270 /
 // 1580).
 static int64_t scores_split_max_wgs(const Problem& pr) {
   const int64_t m = pr.M, n = pr.N;
-  return n >= 64 * m ? 256 : n >= 8 * m ? 128 : n >= 2 * m && n >= 2048 ? 32 : 0;
+  if (n < 2048) return 0;
+  return n >= 64 * m ? 256 : n >= 8 * m ? 128 : n >= 2 * m && n >= 4096 ? 32 : 0;
 }
+// Most query rows of a KV head's group for the finer key splits.
+constexpr int64_t kFewRows = 32;
 // Bytes of the fp32 partials of a plan (O, offset, weight sum, row sum).
 size_t split_bytes(const Problem& pr, const SplitPlan& sp) {
   const size_t rows = (size_t)pr.B * pr.H * sp.nsplit * sp.mpad;
@@ -419,18 +425,95 @@ SplitPlan split_plan(const Problem& pr, bool top_left, int64_t max_wgs = 255,
   int64_t hi = pr.N;
   if (pr.causal) hi = std::min<int64_t>(pr.N, std::max<int64_t>(0, off + pr.M));
   const int64_t nt = (hi + 63) / 64;
-  for (int64_t want = std::min<int64_t>((512 + wgs - 1) / wgs, nt / 8); want >= 2; --want) {
+  const bool few = (int64_t)pr.G * pr.M <= kFewRows;
+  // Partials are indexed by (head, split, position): M rounded up.
+  const int64_t unit = few ? kFewRows : fas::kFwdRows;
+  for (int64_t want = std::min<int64_t>((512 + wgs - 1) / wgs, nt / (few ? 2 : 8)); want >= 2;
+       --want) {
     const int64_t tps = (nt + want - 1) / want;
     const int64_t ns = (nt + tps - 1) / tps;
     if (ns < 2) break;
     SplitPlan c;
     c.nsplit = (int)ns;
-    c.tps = (int)tps;
-    // Partials are indexed by (head, split, position): M rounded up.
-    c.mpad = (((int64_t)pr.M + fas::kFwdRows - 1) / fas::kFwdRows) * fas::kFwdRows;
+    c.mpad = (((int64_t)pr.M + unit - 1) / unit) * unit;
     if (split_bytes(pr, c) <= max_bytes) return c;
   }
   return sp;
+}
+
+// How a plain or row-sum forward runs: rows per workgroup (256, or 128 with
+// the key tiles split between wave pairs) and workgroups per row block (key
+// split, 256 rows only).
+struct FwdPlan {
+  int bm = fas::kFwdRows, nsplit = 1, tps = 0;
+};
+// The estimated end of each choice in steps of one 64-key tile per wave
+// (about 2 us at D = 128, 1 below), one workgroup at a time per CU:
+//  * row blocks start longest first, so one round ends with the longest, two
+//    with the longest or with the last of the first round and the first of
+//    the second; never before the mean over the CUs;
+//  * a workgroup costs about 2.5 steps besides its tiles (q and first K/V
+//    loads, epilogue), 3 with the merge of the 128-row blocks;
+//  * steps of the 128-row blocks move twice the K/V bytes per row, and a chip
+//    that runs evenly loaded clocks lower than one waiting for its longest
+//    row blocks: they count 1.35;
+//  * a key split adds the combine kernel: about 6 us, and its partials
+//    written and read back at 5 TB/s.
+// Measured (us, row-sum calls; 256 rows / 128 rows / split in two or eight):
+// B1 H32 S1024 D128 causal 34.3 / 24.1; S2048 59.9 / 49.2; S4096 147 / 168;
+// B1 H16 S4096 108 / 83; B1 H16 S2048 57.8 / 36.9 / 47.5; B2 H16 S1531 D64
+// full 33.7 / 40.1 / 49.4, causal 33.8 / 23.9; B1 H32/8 M200 N8000 195 / 111
+// / 45.4 (61.2 as 14 splits in two rounds); B1 H32 M256 N16384 388 / 236 /
+// 91.4 (105 as 16 splits in two rounds).
+FwdPlan fwd_plan(const Problem& pr, int pack, bool top_left, const SplitPlan& cap) {
+  FwdPlan best;
+  const int64_t cus = kCus, groups = (int64_t)pr.B * (pr.H / pack);
+  const int64_t n256 = groups * (((int64_t)pr.M * pack + 255) / 256);
+  if (n256 == 0 || pr.N == 0 || n256 > 2 * cus) return best;
+  const int64_t off = top_left ? 0 : (int64_t)pr.N - pr.M;
+  // Steps of row block rb: its key tiles, or pairs of them.
+  auto steps = [&](int64_t bm, int64_t rb) {
+    int64_t hi = pr.N;
+    if (pr.causal) {
+      const int64_t last = std::min<int64_t>(pr.M, (bm * (rb + 1) - 1) / pack + 1);
+      hi = std::min<int64_t>(pr.N, std::max<int64_t>(0, off + last));
+    }
+    const int64_t tiles = (hi + 63) / 64;
+    return bm == 256 ? tiles : (tiles + 1) / 2;
+  };
+  auto makespan = [&](int64_t bm, double over) {
+    const int64_t nrb = ((int64_t)pr.M * pack + bm - 1) / bm, n = groups * nrb;
+    auto at = [&](int64_t i) { return (double)steps(bm, nrb - 1 - i / groups) + over; };
+    double sum = 0;
+    for (int64_t rb = 0; rb < nrb; ++rb) sum += (double)steps(bm, rb) + over;
+    double end = std::max(at(0), sum * (double)groups / (double)cus);
+    if (n > cus) end = std::max(end, at(cus - 1) + at(cus));
+    return end;
+  };
+  double cost = makespan(256, 2.5);
+  if (n256 <= cus) {
+    const double c = 1.35 * makespan(128, 3.0);
+    if (c < cost) {
+      cost = c;
+      best.bm = 128;
+    }
+  }
+  const int64_t nt = steps(256, ((int64_t)pr.M * pack + 255) / 256 - 1);
+  const double us_per_step = pr.D == 128 ? 2.0 : 1.0;
+  for (int64_t want = 2; want <= cap.nsplit; ++want) {
+    const int64_t tps = (nt + want - 1) / want, ns = tps > 0 ? (nt + tps - 1) / tps : 0;
+    if (ns != want) continue;
+    const double partials = (double)pr.B * pr.H * pr.M * (double)ns * (pr.D + 3) * 8;
+    const double c = (double)((n256 * ns + cus - 1) / cus) * ((double)tps + 2.5) +
+                     (6.0 + partials / 5e6) / us_per_step;
+    if (c < cost) {
+      cost = c;
+      best.bm = 256;
+      best.nsplit = (int)ns;
+      best.tps = (int)tps;
+    }
+  }
+  return best;
 }
 
 // Whether a variant's forward pass is the plain or row-sum kernel (the ones
@@ -657,13 +740,15 @@ T* at(void* ws, size_t off) {
   return reinterpret_cast<T*>(static_cast<char*>(ws) + off);
 }
 
-// Points the forward at its key-split partials when the plan splits.
-void apply_split(fas::FwdParams& p, const Workspace& w, void* ws) {
-  if (!w.has_split) return;
-  const SplitPlan& sp = w.sp;
-  p.nsplit = sp.nsplit;
-  p.tps = sp.tps;
-  p.Mpad = (int)sp.mpad;
+// Row blocks and key split of a plain or row-sum forward, with its partials.
+void apply_plan(fas::FwdParams& p, const Problem& pr, bool top_left, const Workspace& w, void* ws) {
+  const FwdPlan f = fwd_plan(pr, p.pack, top_left, w.sp);
+  p.bm = f.bm;
+  p.nrb = (int)(((int64_t)pr.M * p.pack + f.bm - 1) / f.bm);
+  if (f.nsplit == 1) return;
+  p.nsplit = f.nsplit;
+  p.tps = f.tps;
+  p.Mpad = (int)w.sp.mpad;
   p.part_o = at<float>(ws, w.so);
   p.part_m = at<float>(ws, w.sm);
   p.part_l = at<float>(ws, w.sl);
@@ -692,7 +777,7 @@ int run_raw(const char* fn, int variant, const fas_attn_args* a, int64_t split, 
 
   // Attention output.
   fas::FwdParams p = fwd_params(a, pr, cross, fas::kFwdRows);
-  apply_split(p, w, ws);
+  apply_plan(p, pr, cross, w, ws);
   if ((rc = run_fwd(fn, p, pr, fas::kFwdPlain, stream))) return rc;
   if (pr.M == 0) return zero_out3(fn, out, st, pr.B, pr.Hk, ncols, stream);
 
@@ -743,7 +828,7 @@ int run_softmax(const char* fn, int variant, const fas_attn_args* a, int64_t spl
     p.zero_words = at<uint32_t>(ws, w.ticket);
     p.n_zero_words = (int)(w.cp.ngroups * w.cp.nunits);
   }
-  if (!buffered) apply_split(p, w, ws);
+  if (!buffered) apply_plan(p, pr, false, w, ws);
   if (buffered) {
     p.region = at<uint16_t>(ws, w.region);
     p.region_m = at<float>(ws, w.region_m);
@@ -973,7 +1058,7 @@ static int attention_with_scores_impl(const fas_attn_args* a, void* scores, cons
     // scores-only kernel writes the masked scores in parallel over keys.
     fas::FwdParams p = fwd_params(a, pr, false, fas::kFwdRows);
     rescale_dropout(p, a);
-    apply_split(p, w, ws);
+    apply_plan(p, pr, false, w, ws);
     if ((rc = run_fwd(fn, p, pr, fas::kFwdPlain, stream))) return rc;
     return run_scores(fn, a, pr, scores, st, true, stream);
   }
@@ -1062,7 +1147,7 @@ int fas_attention_with_row_sum(const fas_attn_args* a, float* row_sum, const int
   const Workspace w = layout(FAS_VARIANT_ROW_SUM, pr, 0);
   if ((rc = check_workspace(fn, w, ws, ws_bytes))) return rc;
   fas::FwdParams p = fwd_params(a, pr, false, fas::kFwdRows);
-  apply_split(p, w, ws);
+  apply_plan(p, pr, false, w, ws);
   p.aux = row_sum;
   p.sa0 = st[0];
   p.sa1 = st[1];
@@ -1146,7 +1231,7 @@ int fas_attention_forward(const fas_attn_args* a, float* lse, const int64_t st[3
   if ((rc = check_keep(fn, a, pr, &kl))) return rc;
   fas::FwdParams p = fwd_params(a, pr, false, fas::kFwdRows);
   rescale_dropout(p, a);
-  apply_split(p, w, ws);
+  apply_plan(p, pr, false, w, ws);
   p.lse_ln = lse;
   p.sl0 = st[0];
   p.sl1 = st[1];

@@ -270,8 +270,10 @@ template <class E, int D, int MODE, int NW, bool DROP, bool PACK, bool KS2 = fal
 __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(NW == 4 ? 1 : 2, 2)))
 void fwd_kernel(const FwdParams p) {
   static_assert(MODE != kFwdScores || NW == 8 || NW == 4, "the score writer uses 4 or 8 waves");
-  static_assert(!KS2 || (MODE == kFwdScores && !DROP && !PACK),
+  static_assert(!KS2 || !(MODE == kFwdScores && (DROP || PACK)),
                 "the key-split writer is the unpacked score writer");
+  static_assert(!KS2 || MODE != kFwdRegion,
+                "modes with key-split instances");
   static_assert(ALN || MODE == kFwdScores, "only the score writer has unaligned rows");
   constexpr int NH = NW / 2;  // score writer: loader waves [0, NH), storer waves [NH, NW)
   const int pack = PACK ? p.pack : 1;
@@ -291,7 +293,7 @@ void fwd_kernel(const FwdParams p) {
   // every global store instruction writes 8 full 128-byte row segments:
   // 2 stages x NH loader tiles, then one tile per storer (kMid: one stage of
   // loader tiles, handed over within the step).
-  constexpr bool kMid = KS2 && NW == 8;
+  constexpr bool kMid = kSplit && KS2 && NW == 8;
   constexpr int TSZ = 256;  // 16-byte units per wave tile
   constexpr int SG = kSplit ? (kMid ? 2 : 3) * NH * TSZ : 1;
   constexpr int kLoaderStg = kMid ? 1 : 2;  // stages of loader tiles
@@ -303,7 +305,7 @@ void fwd_kernel(const FwdParams p) {
   // weight sums pass through the same LDS, which is sized for the larger.
   union KvLds {
     uint16_t t[2][NTS][2][TILE];
-    float merge[KS2 ? NH * (DB * 16 + 2) * 64 : 1];
+    float merge[KS2 ? NH * (DB * 16 + 3) * 64 : 1];
   };
   __shared__ __attribute__((aligned(16))) KvLds kv_lds;
   auto& kv = kv_lds.t;
@@ -326,13 +328,14 @@ void fwd_kernel(const FwdParams p) {
   const bool loader = !kSplit || wave < NH;
   // The wave's 32-row slice of the row block, and (KS2) its key-tile parity.
   const int slice = KS2 ? (wave & (NH - 1)) : wave;
-  const int kpar = KS2 && !loader ? 1 : 0;
+  const int kpar = KS2 && wave >= NH ? 1 : 0;
   if (blockIdx.x == 0 && p.zero_words != nullptr)
     for (int i = tid; i < p.n_zero_words; i += NW * 64) p.zero_words[i] = 0u;
 
   // Split over keys: the plain and row-sum modes may give a row block to
   // nsplit workgroups, each over its own share of the key tiles.
-  constexpr bool kCanSplit = MODE == kFwdPlain || MODE == kFwdPlainKeepBits || MODE == kFwdRowSum;
+  constexpr bool kCanSplit =
+      !KS2 && (MODE == kFwdPlain || MODE == kFwdPlainKeepBits || MODE == kFwdRowSum);
   int rb, grp, split = 0;
   {
     int bid = blockIdx.x;
@@ -787,7 +790,7 @@ void fwd_kernel(const FwdParams p) {
   // non-causal one): the step's score stores go between the O += P V MFMAs,
   // where the zero batches would be, and the S MFMAs run without stores.
   auto main_loop = [&](auto role, auto nz_tag) __attribute__((always_inline)) {
-    constexpr bool ST = decltype(role)::value;
+    constexpr bool ST = kSplit && decltype(role)::value;
     constexpr bool NZ = ST && decltype(nz_tag)::value;
 
     // One key tile; the LDS stage is a compile-time constant, so the
@@ -798,11 +801,11 @@ void fwd_kernel(const FwdParams p) {
     auto step = [&](int it, auto stage_tag, auto mask_tag) __attribute__((always_inline)) {
       constexpr int stage = decltype(stage_tag)::value;
       constexpr bool MK = decltype(mask_tag)::value;
-      // KS2: the storers (the ST copy; KS2 launches always have storers)
-      // take the odd tiles.  A compile-time slot keeps the LDS operand
-      // addresses of the two roles apart; with the slot a runtime value
-      // every address carried it and the storer's loop spilled.
-      constexpr int kp = KS2 && ST ? 1 : 0;
+      // KS2: the upper waves (the score writer's storers) take the odd
+      // tiles.  A compile-time slot keeps the LDS operand addresses of the
+      // two roles apart; with the slot a runtime value every address carried
+      // it and the storer's loop spilled.
+      constexpr int kp = KS2 && decltype(role)::value ? 1 : 0;
       const int tw = NTS * it + kp;  // this wave's key tile
       const bool masked = MK && tw >= tfull;
       if (it + 1 < t_end) issue_tile(it + 1, stage ^ 1);
@@ -1085,6 +1088,11 @@ void fwd_kernel(const FwdParams p) {
     } else {
       main_loop(std::false_type{}, std::false_type{});
     }
+  } else if constexpr (KS2) {
+    if (kpar)
+      main_loop(std::true_type{}, std::false_type{});
+    else
+      main_loop(std::false_type{}, std::false_type{});
   } else {
     main_loop(std::false_type{}, std::false_type{});
   }
@@ -1109,21 +1117,22 @@ void fwd_kernel(const FwdParams p) {
   }
 
   if constexpr (KS2) {
-    // The storer's partial O, offset and weight sum meet its loader's in LDS
-    // (the K/V tiles' space, free after the loop); lane l of both holds the
-    // same row and head dims.
-    float* mb = kv_lds.merge + slice * (DB * 16 + 2) * 64;
+    // The upper wave's partial O, offset and weight sum (and row sum) meet
+    // the lower wave's in LDS (the K/V tiles' space, free after the loop);
+    // lane l of both holds the same row and head dims.
+    float* mb = kv_lds.merge + slice * (DB * 16 + 3) * 64;
     lds_barrier();
-    if (!loader) {
+    if (kpar) {
 #pragma unroll
       for (int db = 0; db < DB; ++db)
 #pragma unroll
         for (int r = 0; r < 16; ++r) mb[(db * 16 + r) * 64 + lane] = oacc[db][r];
       mb[DB * 16 * 64 + lane] = m_ref;
       mb[(DB * 16 + 1) * 64 + lane] = l_i;
+      if constexpr (MODE == kFwdRowSum) mb[(DB * 16 + 2) * 64 + lane] = rsum;
     }
     lds_barrier();
-    if (!loader) return;
+    if (kpar) return;
     const float mo = mb[DB * 16 * 64 + lane], lo = mb[(DB * 16 + 1) * 64 + lane];
     const float mn = fmaxf(m_ref, mo);
     const float a0 = m_ref == neg_inf() ? 0.f : exp2f_fast((m_ref - mn) * p.qk_scale);
@@ -1135,6 +1144,7 @@ void fwd_kernel(const FwdParams p) {
         oacc[db][r] = oacc[db][r] * a0 + mb[(db * 16 + r) * 64 + lane] * a1;
     l_i = l_i * a0 + lo * a1;
     m_ref = mn;
+    if constexpr (MODE == kFwdRowSum) rsum += mb[(DB * 16 + 2) * 64 + lane];
   }
   // Epilogue: O = acc / l, base-2 LSE, row sums.
   const float l_tot = xor32_add(l_i);
@@ -1259,7 +1269,8 @@ __global__ __launch_bounds__(256) void fwd_combine_kernel(const FwdParams p) {
 
 template <class E, int D, int MODE, int NW, bool DROP, bool PACK, bool KS2 = false, bool ALN = true>
 hipError_t launch_fwd_t(const FwdParams& p, hipStream_t stream) {
-  constexpr bool kCanSplit = MODE == kFwdPlain || MODE == kFwdPlainKeepBits || MODE == kFwdRowSum;
+  constexpr bool kCanSplit =
+      !KS2 && (MODE == kFwdPlain || MODE == kFwdPlainKeepBits || MODE == kFwdRowSum);
   const int64_t nsplit = kCanSplit ? p.nsplit : 1;
   const dim3 grid((unsigned)((int64_t)p.nrb * (p.B * p.H / p.pack) * nsplit)), block(NW * 64);
   hipLaunchKernelGGL((fwd_kernel<E, D, MODE, NW, DROP, PACK, KS2, ALN>), grid, block, 0, stream, p);

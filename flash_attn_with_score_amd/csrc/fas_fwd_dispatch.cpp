@@ -8,6 +8,7 @@ hipError_t launch_fwd_rowsum(const FwdParams& p, int dtype, int d, hipStream_t s
 hipError_t launch_fwd_scores(const FwdParams& p, int dtype, int d, hipStream_t s);
 hipError_t launch_fwd_scores_unaligned(const FwdParams& p, int dtype, int d, hipStream_t s);
 hipError_t launch_fwd_region(const FwdParams& p, int dtype, int d, hipStream_t s);
+hipError_t launch_fwd_key_split(const FwdParams& p, int mode, int dtype, int d, hipStream_t s);
 hipError_t launch_fwd_dropout(const FwdParams& p, int mode, int dtype, int d, hipStream_t s);
 hipError_t launch_fwd_packed(const FwdParams& p, int mode, int dtype, int d, hipStream_t s);
 hipError_t launch_fwd_scores_packed(const FwdParams& p, int dtype, int d, hipStream_t s);
@@ -15,11 +16,16 @@ hipError_t launch_fwd_scores_packed(const FwdParams& p, int dtype, int d, hipStr
 // GQA-packed launches (p.pack > 1) take their own instances; the host never
 // packs a launch with dropout.
 hipError_t launch_fwd(const FwdParams& p, int mode, int dtype, int d, hipStream_t s) {
-  // Only the unpacked score writer without dropout has 128- and 64-row
-  // instances; every other launch is built for 256-row blocks.
-  const bool small_writer = mode == kFwdScores && p.pack == 1 && !p.dropout &&
-                            (p.bm == kFwdRows / 2 || p.bm == kFwdRows / 4);
-  if (p.bm != kFwdRows && !small_writer) return hipErrorInvalidValue;
+  // Row blocks below 256: the unpacked score writer without dropout (128 and
+  // 64 rows) and, without a key split over workgroups, the plain and row-sum
+  // modes (128 rows).
+  if (p.bm != kFwdRows) {
+    if (mode == kFwdScores
+            ? p.dropout || p.pack != 1 || (p.bm != kFwdRows / 2 && p.bm != kFwdRows / 4)
+            : mode == kFwdRegion || p.bm != kFwdRows / 2 || p.nsplit != 1)
+      return hipErrorInvalidValue;
+    if (mode != kFwdScores && !p.dropout) return launch_fwd_key_split(p, mode, dtype, d, s);
+  }
   if (mode == kFwdScores && !p.scores_aligned) {
     if (p.pack > 1 && p.dropout) return hipErrorInvalidValue;
     return launch_fwd_scores_unaligned(p, dtype, d, s);

@@ -5,7 +5,11 @@
 
 namespace fas {
 
+hipError_t launch_fwd_dropout_key_split(const FwdParams& p, int mode, int dtype, int d,
+                                        hipStream_t s);
+
 hipError_t launch_fwd_dropout(const FwdParams& p, int mode, int dtype, int d, hipStream_t s) {
+  if (p.bm == 128) return launch_fwd_dropout_key_split(p, mode, dtype, d, s);
   switch (mode) {
     case kFwdPlain: return launch_fwd_mode<kFwdPlain, 8, true>(p, dtype, d, s);
     case kFwdPlainKeepBits: return launch_fwd_mode<kFwdPlainKeepBits, 8, true>(p, dtype, d, s);
