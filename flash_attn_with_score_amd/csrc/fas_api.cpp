@@ -530,12 +530,54 @@ int64_t bwd_mpad(const Problem& pr) {
   return (((int64_t)pr.M + fas::kBwdBlock - 1) / fas::kBwdBlock) * fas::kBwdBlock;
 }
 int64_t bwd_nkb(const Problem& pr) { return ((int64_t)pr.N + fas::kBwdBlock - 1) / fas::kBwdBlock; }
-// The dK/dV kernel walks a KV head's whole query-head group per workgroup
-// unless that leaves fewer workgroups than the chip has CUs; then it takes
-// one query head per workgroup and writes fp32 partials.
-bool bwd_partial(const Problem& pr) {
+// Workgroups per key block and KV head of the dK/dV kernel: each walks a
+// share of the row tiles (64 rows, G heads) that see the block.  With one, the
+// causal mask's first key blocks set the end wherever all run in one round
+// (B1 H32/8 S4096 D128: 256 workgroups of 4 to 256 tiles, 619 us; in two
+// pieces 395 us and 14 us to reduce), and few KV heads leave CUs idle.  More cost fp32 partials,
+// written and read once (5 TB/s), about 6 us for the reduction, and about 3
+// tiles for each further workgroup's K and V loads and stores.  Estimated as
+// the forward's plan: the longest, or the mean over the CUs; at least 4 tiles
+// a piece for the longest block, at most 8 pieces, or G where the workspace
+// holds G partials.
+bool bwd_per_head(const Problem& pr) {
   return pr.G > 1 && (int64_t)pr.B * pr.Hk * bwd_nkb(pr) < 256;
 }
+int bwd_pieces(const Problem& pr) {
+  const int64_t nkb = bwd_nkb(pr), heads = (int64_t)pr.B * pr.Hk, n = heads * nkb;
+  const int64_t rows = (pr.M + 63) / 64;
+  if (n == 0 || rows == 0) return 1;
+  auto tiles = [&](int64_t kb) {
+    const int64_t lo = pr.causal
+        ? std::max<int64_t>(0, fas::kBwdBlock * kb - ((int64_t)pr.N - pr.M)) / 64 : 0;
+    return std::max<int64_t>(0, rows - lo) * pr.G;
+  };
+  const int64_t slots = pr.D == 128 ? kCus : 2 * kCus;  // one wave per SIMD, or two
+  const double us_per_tile = pr.D == 128 ? 2.4 : 2.0;
+  if (n > 4 * slots) return 1;
+  double sum = 0;
+  for (int64_t kb = 0; kb < nkb; ++kb) sum += (double)(heads * tiles(kb));
+  int best = 1;
+  double cost = 1e30;
+  const int most = bwd_per_head(pr) ? std::min(8, pr.G) : 8;
+  for (int s = 1; s <= most; ++s) {
+    if (s > 1 && tiles(0) < 4 * s) break;
+    const double longest = (double)((tiles(0) + s - 1) / s) + 3.0;
+    double c = std::max(longest, (sum + 3.0 * (double)(n * s)) / (double)slots);
+    // Blocks of equal length run in whole rounds.
+    if (!pr.causal) c = longest * (double)((n * s + slots - 1) / slots);
+    if (s > 1)
+      c += (6.0 + (double)heads * pr.N * s * 2 * pr.D * 8 / 5e6) / us_per_tile;
+    if (c < cost) {
+      cost = c;
+      best = s;
+    }
+  }
+  return best;
+}
+// Partials the workspace holds: the launch's pieces, or one per query head
+// wherever G > 1 and B*Hk*nkb is below 256.
+int bwd_part_count(const Problem& pr) { return bwd_per_head(pr) ? pr.G : bwd_pieces(pr); }
 // The backward's stored dS (BwdParams.ds): 32-row block r sees 32-key blocks
 // [0, clamp(r + a, 0, ceil(N/32))): a = floor((N - M + 31) / 32) + 1 under the
 // causal mask (block (r, j) holds a visible pair iff (N - M) + 32 r + 31 >=
@@ -666,10 +708,10 @@ Workspace layout(int variant, const Problem& pr, int64_t split, size_t budget = 
     off += align256(rows);
     w.delta = off;
     off += align256(rows);
-    if (bwd_partial(pr)) {
+    if (bwd_part_count(pr) > 1) {
       w.has_part = true;
       w.part = off;
-      off += align256((size_t)pr.B * pr.H * pr.N * 2 * pr.D * 4);
+      off += align256((size_t)pr.B * pr.Hk * bwd_part_count(pr) * pr.N * 2 * pr.D * 4);
     }
     // dS for the dQ kernel (2 bytes per visible pair, in 32 x 32 blocks),
     // when a head's blocks stay below 2 GiB, all of them within
@@ -1351,7 +1393,7 @@ int fas_attention_backward(const fas_attn_args* a, const void* dout, const int64
   p.nkb = (int)bwd_nkb(pr);
   p.nrb = p.Mpad / fas::kBwdBlock;
   p.nprep = (p.Mpad + (2048 / pr.D) - 1) / (2048 / pr.D);
-  p.partial = bwd_partial(pr) ? 1 : 0;
+  p.pieces = bwd_pieces(pr);
   p.n32 = (pr.N + 31) / 32;
   if (w.has_bits) p.drop_bits = at<uint32_t>(ws, w.bits);
   if (w.has_ds) {

@@ -16,7 +16,7 @@ static hipError_t bwd_t(const BwdParams& p, hipStream_t s) {
     hipLaunchKernelGGL((bwd_prep_kernel<E, D>), dim3((unsigned)(bh * p.nprep)), dim3(256), 0, s,
                        p);
   if (p.N > 0) {
-    const int64_t rest = p.partial ? bh : (int64_t)p.B * p.Hk;
+    const int64_t rest = (int64_t)p.B * p.Hk * p.pieces;
     const dim3 grid((unsigned)(rest * p.nkb));
     if (!p.dropout)
       hipLaunchKernelGGL((bwd_dkdv_kernel<E, D, 0>), grid, dim3(256), 0, s, p);
@@ -24,7 +24,7 @@ static hipError_t bwd_t(const BwdParams& p, hipStream_t s) {
       hipLaunchKernelGGL((bwd_dkdv_kernel<E, D, 2>), grid, dim3(256), 0, s, p);
     else
       hipLaunchKernelGGL((bwd_dkdv_kernel<E, D, 1>), grid, dim3(256), 0, s, p);
-    if (p.partial) {
+    if (p.pieces > 1) {
       const int64_t total = (int64_t)p.B * p.Hk * p.N * (D / 8);
       int64_t blocks = (total + 255) / 256;
       if (blocks > 16384) blocks = 16384;

@@ -18,10 +18,12 @@
 //                     row-major tiles with the transposing LDS load.  GQA: a
 //                     workgroup walks every query head of its KV group, so dK
 //                     and dV are summed over the group in fp32 (the reference
-//                     sums per-head fp16 results, flash.py:258-259).  When
-//                     that leaves too few workgroups for the chip, each
-//                     workgroup takes one query head and writes fp32 partials
-//                     that bwd_dkdv_reduce_kernel adds in head order.
+//                     sums per-head fp16 results, flash.py:258-259).  A key
+//                     block's row tiles (of all its heads) may be dealt to
+//                     several workgroups, so that the chip is full and a
+//                     causal mask's long key blocks do not set the end; they
+//                     write fp32 partials that bwd_dkdv_reduce_kernel adds in
+//                     order.
 //   bwd_dq_kernel     query-block outer (flash.py:758-918), the forward pass's
 //                     data flow: a wave owns 32 rows, holds their Q and dO as B
 //                     operands, and streams 64-key tiles of K and V:
@@ -103,8 +105,11 @@ __global__ __launch_bounds__(256) void bwd_prep_kernel(const BwdParams p) {
 // the dP accumulator then starts at 0 and delta is added afterwards.  DROP 1
 // evaluates Z (Philox) and, with drop_bits, stores it for the dQ kernel;
 // DROP 2 reads the forward's keep words (keep_keys) and has no Philox code.
+// Two waves per SIMD up to D = 64 (left free, D = 64 took 258 registers, one
+// wave per SIMD).
 template <class E, int D, int DROP>
-__global__ __launch_bounds__(256) void bwd_dkdv_kernel(const BwdParams p) {
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D <= 64 && DROP != 1 ? 2 : 1)))
+void bwd_dkdv_kernel(const BwdParams p) {
   constexpr int KS = D / 16;               // k-steps over the head dim
   constexpr int DB = D >= 32 ? D / 32 : 1;  // 32-dim blocks of dK^T / dV^T
   constexpr int NW = 4;
@@ -120,21 +125,13 @@ __global__ __launch_bounds__(256) void bwd_dkdv_kernel(const BwdParams p) {
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lane = tid & 63, c = lane & 31, g = lane >> 5;
-  // Key blocks ascending (for causal masks, the longest first).
-  const int nrest = p.partial ? p.B * p.H : p.B * p.Hk;
+  // Key blocks ascending (for causal masks, the longest first), then the
+  // pieces of each KV head's row tiles.
+  const int nrest = p.B * p.Hk * p.pieces;
   const int kb = blockIdx.x / nrest, rest = blockIdx.x % nrest;
-  int b, hk, h0, nheads;
-  if (p.partial) {
-    b = rest / p.H;
-    h0 = rest % p.H;
-    hk = h0 / p.G;
-    nheads = 1;
-  } else {
-    b = rest / p.Hk;
-    hk = rest % p.Hk;
-    h0 = hk * p.G;
-    nheads = p.G;
-  }
+  const int piece = rest % p.pieces, bhk = rest / p.pieces;
+  const int b = bhk / p.Hk, hk = bhk % p.Hk;
+  const int h0 = hk * p.G;
   const int key0 = kb * BK + 32 * wave;  // this wave's keys [key0, key0 + 32)
 
   // K and V (B operands of S = Q K^T and dP = dO V^T): lane holds row key0 + c,
@@ -160,7 +157,10 @@ __global__ __launch_bounds__(256) void bwd_dkdv_kernel(const BwdParams p) {
 
   // Query rows that can see a key of the block.
   const int rstart = p.causal ? max(0, kb * BK - p.causal_off) : 0;
-  const int t0 = rstart / TQ, t1 = (p.M + TQ - 1) / TQ;
+  const int tlo = rstart / TQ, tiles = max(0, (p.M + TQ - 1) / TQ - tlo);
+  // This piece's tiles [s0, s1) of the G heads' tiles in head order.
+  const int64_t steps = (int64_t)p.G * tiles;
+  const int s0 = (int)(steps * piece / p.pieces), s1 = (int)(steps * (piece + 1) / p.pieces);
   const float qk = p.qk_scale;
   const uint32_t q_base = lds_addr(&qlds[0][0]), g_base = lds_addr(&glds[0][0]);
 
@@ -170,7 +170,9 @@ __global__ __launch_bounds__(256) void bwd_dkdv_kernel(const BwdParams p) {
   constexpr bool from_keys = DROP == 2;
   const bool bits = DROP == 1 && p.drop_bits != nullptr;
   const int r32 = (p.M + 31) >> 5;
-  for (int hh = 0; hh < nheads && t0 < t1; ++hh) {
+  for (int hh = 0; hh < p.G; ++hh) {
+    const int t0 = tlo + max(0, s0 - hh * tiles), t1 = tlo + min(tiles, s1 - hh * tiles);
+    if (t0 >= t1) continue;
     const int h = h0 + hh;
     const int64_t bh = (int64_t)b * p.H + h;
     __amdgpu_buffer_rsrc_t rbits = make_rsrc(p.drop_bits, 0), rkeys = rbits;
@@ -387,7 +389,7 @@ __global__ __launch_bounds__(256) void bwd_dkdv_kernel(const BwdParams p) {
 #pragma unroll
     for (int db = 0; db < DB; ++db) dv[db] *= p.drop.scale;
   }
-  if (!p.partial) {
+  if (p.pieces == 1) {
     uint16_t* dkr = p.dk + b * p.sdk0 + hk * p.sdk1 + (int64_t)key * p.sdk2;
     uint16_t* dvr = p.dv + b * p.sdv0 + hk * p.sdv1 + (int64_t)key * p.sdv2;
 #pragma unroll
@@ -402,7 +404,7 @@ __global__ __launch_bounds__(256) void bwd_dkdv_kernel(const BwdParams p) {
         }
       }
   } else {
-    float* pr = p.part + (((int64_t)b * p.H + h0) * p.N + key) * (2 * D);
+    float* pr = p.part + (((int64_t)bhk * p.pieces + piece) * p.N + key) * (2 * D);
 #pragma unroll
     for (int db = 0; db < DB; ++db)
 #pragma unroll
@@ -424,8 +426,8 @@ __global__ __launch_bounds__(256) void bwd_dkdv_kernel(const BwdParams p) {
   }
 }
 
-// dK, dV of KV head hk = sum over its G query heads of the fp32 partials, in
-// head order; one thread per 8 elements.
+// dK, dV of a KV head = sum of its pieces' fp32 partials, in order; one
+// thread per 8 elements.
 template <class E, int D>
 __global__ __launch_bounds__(256) void bwd_dkdv_reduce_kernel(const BwdParams p) {
   constexpr int CPR = D / 8;
@@ -438,12 +440,19 @@ __global__ __launch_bounds__(256) void bwd_dkdv_reduce_kernel(const BwdParams p)
     const int64_t bhk = r / p.N;
     const int hk = (int)(bhk % p.Hk), b = (int)(bhk / p.Hk);
     float a[8] = {}, v[8] = {};
-    for (int j = 0; j < p.G; ++j) {
-      const float* src = p.part + (((int64_t)b * p.H + hk * p.G + j) * p.N + key) * (2 * D) + 8 * ch;
+#pragma unroll 4
+    for (int j = 0; j < p.pieces; ++j) {
+      const float* src = p.part + ((bhk * p.pieces + j) * p.N + key) * (2 * D) + 8 * ch;
+      const f32x4 a0 = *reinterpret_cast<const f32x4*>(src);
+      const f32x4 a1 = *reinterpret_cast<const f32x4*>(src + 4);
+      const f32x4 v0 = *reinterpret_cast<const f32x4*>(src + D);
+      const f32x4 v1 = *reinterpret_cast<const f32x4*>(src + D + 4);
 #pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        a[e] += src[e];
-        v[e] += src[D + e];
+      for (int e = 0; e < 4; ++e) {
+        a[e] += a0[e];
+        a[4 + e] += a1[e];
+        v[e] += v0[e];
+        v[4 + e] += v1[e];
       }
     }
     const int d0 = 8 * ch;

@@ -191,7 +191,7 @@ struct BwdParams {
   uint16_t* dq;
   uint16_t* dk;
   uint16_t* dv;
-  float* part;           // workspace (B*H, N, 2D) fp32 per-query-head dK | dV (partial mode)
+  float* part;           // workspace (B*Hk, pieces, N, 2D) fp32 dK | dV partials (pieces > 1)
   int64_t sq0, sq1, sq2;
   int64_t sk0, sk1, sk2;
   int64_t sv0, sv1, sv2;
@@ -208,7 +208,7 @@ struct BwdParams {
   int nkb;               // 128-key blocks (dK/dV kernel)
   int nrb;               // 128-row blocks (dQ kernel)
   int nprep;             // row groups per (b, head) of the prep kernel
-  int partial;           // dK/dV kernel: one query head per workgroup, fp32 partials
+  int pieces;            // dK/dV kernel: workgroups per key block and KV head
   float sm_scale;        // |sm_scale|
   float scale_signed;    // sm_scale with its sign: dQ = s sum_j dS_ij k_j, dK = s sum_i dS_ij q_i
   float qk_scale;        // |sm_scale| * log2(e)
