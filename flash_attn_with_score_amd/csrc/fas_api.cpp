@@ -380,6 +380,8 @@ struct Workspace {
   bool has_ds = false;
   size_t so = 0, sm = 0, sl = 0, sr = 0;                        // key-split partials
   bool has_lse = false, has_part = false, has_bsum = false, has_region = false;
+  size_t few = 0;                                               // kept scores (kFwdFewRows)
+  bool has_few = false;
   bool has_split = false;
   SplitPlan sp;  // the forward's key split (nsplit 1: none)
 };
@@ -406,7 +408,14 @@ static int64_t scores_split_max_wgs(const Problem& pr) {
   return n >= 64 * m ? 256 : n >= 8 * m ? 128 : n >= 2 * m && n >= 4096 ? 32 : 0;
 }
 // Most query rows of a KV head's group for the finer key splits.
-constexpr int64_t kFewRows = 32;
+constexpr int64_t kFewRows = fas::kFwdFewMax;
+// Whether a problem has at most that many and runs the forward that keeps
+// their scores (kFwdFewRows): all of a KV head's query heads in one
+// workgroup, no dropout.
+bool few_rows(const Problem& pr) {
+  return (int64_t)pr.G * pr.M <= fas::kFwdFewMax && pr.pack == pr.G && !pr.dropout && pr.N > 0 &&
+         pr.M > 0;
+}
 // Bytes of the fp32 partials of a plan (O, offset, weight sum, row sum).
 size_t split_bytes(const Problem& pr, const SplitPlan& sp) {
   const size_t rows = (size_t)pr.B * pr.H * sp.nsplit * sp.mpad;
@@ -465,7 +474,8 @@ struct FwdPlan {
 // full 33.7 / 40.1 / 49.4, causal 33.8 / 23.9; B1 H32/8 M200 N8000 195 / 111
 // / 45.4 (61.2 as 14 splits in two rounds); B1 H32 M256 N16384 388 / 236 /
 // 91.4 (105 as 16 splits in two rounds).
-FwdPlan fwd_plan(const Problem& pr, int pack, bool top_left, const SplitPlan& cap) {
+FwdPlan fwd_plan(const Problem& pr, int pack, bool top_left, const SplitPlan& cap,
+                 bool key_pairs) {
   FwdPlan best;
   const int64_t cus = kCus, groups = (int64_t)pr.B * (pr.H / pack);
   const int64_t n256 = groups * (((int64_t)pr.M * pack + 255) / 256);
@@ -491,7 +501,7 @@ FwdPlan fwd_plan(const Problem& pr, int pack, bool top_left, const SplitPlan& ca
     return end;
   };
   double cost = makespan(256, 2.5);
-  if (n256 <= cus) {
+  if (key_pairs && n256 <= cus) {
     const double c = 1.35 * makespan(128, 3.0);
     if (c < cost) {
       cost = c;
@@ -669,7 +679,19 @@ Workspace layout(int variant, const Problem& pr, int64_t split, size_t budget = 
     w.has_lse = true;
     w.lse = off;
     off += align256((size_t)pr.B * pr.H * pr.M * 4);
+    // Few query rows: their scores, fp32, kept by the forward for the column
+    // sums (rows padded to whole key tiles), when they fit the budget.
+    if (variant == FAS_VARIANT_SOFTMAX_COL_SUM && few_rows(pr)) {
+      const size_t bytes =
+          align256((size_t)pr.B * pr.H * pr.M * (((size_t)pr.N + 63) / 64 * 64) * 4);
+      if (off + bytes <= budget) {
+        w.has_few = true;
+        w.few = off;
+        off += bytes;
+      }
+    }
     w.cp = col_plan(pr, variant == FAS_VARIANT_CROSS_SOFTMAX_SUM_BUFFERED, ncols, true);
+    if (w.has_few) w.cp.nsplit = 1;
     if (w.cp.nsplit > 1) {
       // The splits' column sums and one ticket per (output group, unit).
       w.has_part = true;
@@ -783,8 +805,9 @@ T* at(void* ws, size_t off) {
 }
 
 // Row blocks and key split of a plain or row-sum forward, with its partials.
-void apply_plan(fas::FwdParams& p, const Problem& pr, bool top_left, const Workspace& w, void* ws) {
-  const FwdPlan f = fwd_plan(pr, p.pack, top_left, w.sp);
+void apply_plan(fas::FwdParams& p, const Problem& pr, bool top_left, const Workspace& w, void* ws,
+                bool key_pairs = true) {
+  const FwdPlan f = fwd_plan(pr, p.pack, top_left, w.sp, key_pairs);
   p.bm = f.bm;
   p.nrb = (int)(((int64_t)pr.M * p.pack + f.bm - 1) / f.bm);
   if (f.nsplit == 1) return;
@@ -870,7 +893,17 @@ int run_softmax(const char* fn, int variant, const fas_attn_args* a, int64_t spl
     p.zero_words = at<uint32_t>(ws, w.ticket);
     p.n_zero_words = (int)(w.cp.ngroups * w.cp.nunits);
   }
-  if (!buffered) apply_plan(p, pr, false, w, ws);
+  if (!buffered) apply_plan(p, pr, false, w, ws, !w.has_few);
+  if (w.has_few) {
+    p.few = at<float>(ws, w.few);
+    p.few_pitch = (pr.N + 63) / 64 * 64;
+    p.col = out;
+    p.sc0 = st[0]; p.sc1 = st[1]; p.sc2 = st[2];
+    if ((rc = run_fwd(fn, p, pr, fas::kFwdFewRows, stream))) return rc;
+    if ((int64_t)pr.B * pr.H == 0) return FAS_OK;
+    return hip_status(fn, fas::launch_few_cols(p, pr.dtype, pr.D,
+                                               static_cast<hipStream_t>(stream)));
+  }
   if (buffered) {
     p.region = at<uint16_t>(ws, w.region);
     p.region_m = at<float>(ws, w.region_m);
@@ -1100,6 +1133,13 @@ static int attention_with_scores_impl(const fas_attn_args* a, void* scores, cons
     // scores-only kernel writes the masked scores in parallel over keys.
     fas::FwdParams p = fwd_params(a, pr, false, fas::kFwdRows);
     rescale_dropout(p, a);
+    if (few_rows(pr)) {
+      // The forward writes the scores itself: K is read once.
+      apply_plan(p, pr, false, w, ws, false);
+      p.scores = static_cast<uint16_t*>(scores);
+      p.ss0 = st[0]; p.ss1 = st[1]; p.ss2 = st[2];
+      return run_fwd(fn, p, pr, fas::kFwdFewRows, stream);
+    }
     apply_plan(p, pr, false, w, ws);
     if ((rc = run_fwd(fn, p, pr, fas::kFwdPlain, stream))) return rc;
     return run_scores(fn, a, pr, scores, st, true, stream);

@@ -228,6 +228,9 @@ __device__ __forceinline__ void buf_store16_nt(u32x4 v, __amdgpu_buffer_rsrc_t r
   __builtin_amdgcn_raw_buffer_store_b128(v, r, off, soff, kAuxNT);
 }
 
+// A 16-byte vector at any 2-byte address.
+typedef u32x4 __attribute__((aligned(2))) u32x4_any;
+
 // Score stores.  ALN: every row starts on a 64-byte boundary, so a wave's
 // 128-byte row pieces are whole 64-byte halves of a line and stream past the
 // caches (kAuxNT).  Otherwise a row may start at any element: the pieces

@@ -16,6 +16,10 @@
 //               (attention_cross_token_softmax_sum.py:539-552), as fp16
 //               base-2 exponents relative to a per-row, per-tile maximum
 //               (masked -> -inf)
+//   kFwdFewRows kFwdPlain over at most 32 query rows per KV head (decoding): +
+//               the scores of every key, kept raw in fp32 for the column sums
+//               of the softmax weights, or written as the score matrix, so
+//               that no second pass reads K
 //   kFwdPlainKeepBits
 //               kFwdPlain with dropout, + the keep decisions as bits for the
 //               softmax column pass (which then need not evaluate Philox)
@@ -272,7 +276,7 @@ void fwd_kernel(const FwdParams p) {
   static_assert(MODE != kFwdScores || NW == 8 || NW == 4, "the score writer uses 4 or 8 waves");
   static_assert(!KS2 || !(MODE == kFwdScores && (DROP || PACK)),
                 "the key-split writer is the unpacked score writer");
-  static_assert(!KS2 || MODE != kFwdRegion,
+  static_assert(!KS2 || (MODE != kFwdRegion && MODE != kFwdFewRows),
                 "modes with key-split instances");
   static_assert(ALN || MODE == kFwdScores, "only the score writer has unaligned rows");
   constexpr int NH = NW / 2;  // score writer: loader waves [0, NH), storer waves [NH, NW)
@@ -335,7 +339,8 @@ void fwd_kernel(const FwdParams p) {
   // Split over keys: the plain and row-sum modes may give a row block to
   // nsplit workgroups, each over its own share of the key tiles.
   constexpr bool kCanSplit =
-      !KS2 && (MODE == kFwdPlain || MODE == kFwdPlainKeepBits || MODE == kFwdRowSum);
+      !KS2 && (MODE == kFwdPlain || MODE == kFwdPlainKeepBits || MODE == kFwdRowSum ||
+                MODE == kFwdFewRows);
   int rb, grp, split = 0;
   {
     int bid = blockIdx.x;
@@ -906,6 +911,47 @@ void fwd_kernel(const FwdParams p) {
           }
           if (masked) row_end(s, k0);
         }
+        if constexpr (MODE == kFwdFewRows) {
+          // The lane's row against keys k0 + 16 j + 8 g .. + 7: wave 0 alone
+          // holds rows (the workgroup's others only load K and V).
+          if (row_ok) {
+            if (p.few != nullptr) {
+              float* fr = p.few +
+                          ((int64_t)(b * (p.H / p.G) + hk) * p.G * p.M + vrow) * p.few_pitch + k0 +
+                          8 * g;
+#pragma unroll
+              for (int j = 0; j < 4; ++j) {
+                const f32x16& x = s[j >> 1];
+                const int r0 = 8 * (j & 1);
+                *reinterpret_cast<f32x4*>(fr + 16 * j) =
+                    f32x4{x[r0], x[r0 + 1], x[r0 + 2], x[r0 + 3]};
+                *reinterpret_cast<f32x4*>(fr + 16 * j + 4) =
+                    f32x4{x[r0 + 4], x[r0 + 5], x[r0 + 6], x[r0 + 7]};
+              }
+            } else {
+              uint16_t* sr = p.scores + b * p.ss0 + qh * p.ss1 + (int64_t)qpos * p.ss2;
+#pragma unroll
+              for (int j = 0; j < 4; ++j) {
+                const int key = k0 + 16 * j + 8 * g;
+                float y[8];
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                  const float x = s[j >> 1][8 * (j & 1) + e];
+                  y[e] = x == neg_inf() ? 0.f : x * p.sm_scale;
+                }
+                const u32x4 w = {E::pack(y[0], y[1]), E::pack(y[2], y[3]), E::pack(y[4], y[5]),
+                                 E::pack(y[6], y[7])};
+                if (key + 8 <= p.N) {
+                  *reinterpret_cast<u32x4_any*>(sr + key) = w;
+                } else {
+#pragma unroll
+                  for (int e = 0; e < 7; ++e)
+                    if (key + e < p.N) sr[key + e] = (uint16_t)(w[e >> 1] >> (16 * (e & 1)));
+                }
+              }
+            }
+          }
+        }
         if constexpr (MODE == kFwdRowSum) {
           // Masked scores (-inf) count as 0; only the masked loop copy can
           // hold any, so the others add the tile straight (a pairwise tree:
@@ -1217,12 +1263,12 @@ void fwd_kernel(const FwdParams p) {
 // M + log2 l (+inf for rows that saw no key), and the summed row sums.
 // D/8 threads per row, 8 head dims each.
 template <class E, int D, int MODE>
-__global__ __launch_bounds__(256) void fwd_combine_kernel(const FwdParams p) {
+__device__ __forceinline__ void combine_rows(const FwdParams& p, int block) {
   constexpr int CPR = D / 8;
   constexpr int RPB = 256 / CPR;
   const int nblk = (p.M + RPB - 1) / RPB;
-  const int bh = blockIdx.x / nblk;
-  const int row = (blockIdx.x % nblk) * RPB + (int)threadIdx.x / CPR;
+  const int bh = block / nblk;
+  const int row = (block % nblk) * RPB + (int)threadIdx.x / CPR;
   const int ch = (int)threadIdx.x % CPR;
   if (row >= p.M) return;
   const int b = bh / p.H, h = bh % p.H;
@@ -1267,17 +1313,84 @@ __global__ __launch_bounds__(256) void fwd_combine_kernel(const FwdParams p) {
   }
 }
 
+template <class E, int D, int MODE>
+__global__ __launch_bounds__(256) void fwd_combine_kernel(const FwdParams p) {
+  combine_rows<E, D, MODE>(p, blockIdx.x);
+}
+
+// Second pass of kFwdFewRows: col[key] = sum over the G*M rows of a KV head of
+// exp2(s * qk_scale - lse2), from the scores the forward kept (4 G M bytes a
+// key where a pass over K reads 2 D: B8 H32/8 M1 N8191 D128, 98 us with the
+// column pass over K, 8 us here).  With a key split, workgroups
+// [0, ncombine) merge the output rows as fwd_combine_kernel does and the
+// others form the base-2 normalizers themselves, 8 threads a row, so one
+// launch follows the forward.  A workgroup sums 1024 keys, four a thread.
+template <class E, int D>
+__global__ __launch_bounds__(256) void few_cols_kernel(const FwdParams p, int ncombine) {
+  if ((int)blockIdx.x < ncombine) {
+    combine_rows<E, D, kFwdPlain>(p, blockIdx.x);
+    return;
+  }
+  __shared__ float lse[32];
+  const int nkb = (p.N + 1023) >> 10, item = blockIdx.x - ncombine;
+  const int kb = item % nkb, bhk = item / nkb;
+  const int hk = bhk % (p.H / p.G), b = bhk / (p.H / p.G);
+  const int rows = p.G * p.M;  // at most 32
+  const int tid = threadIdx.x, v = tid >> 3, sub = tid & 7;
+  {
+    const int pos = v / p.G, bh = b * p.H + hk * p.G + (v - pos * p.G);
+    float mx = neg_inf(), l = 0.f;
+    if (v < rows) {
+      if (p.nsplit > 1) {
+        const int64_t base = (int64_t)bh * p.nsplit * p.Mpad + pos;
+        for (int sp = sub; sp < p.nsplit; sp += 8)
+          mx = fmaxf(mx, p.part_m[base + (int64_t)sp * p.Mpad]);
+#pragma unroll
+        for (int w = 1; w < 8; w <<= 1) mx = fmaxf(mx, __shfl_xor(mx, w));
+        for (int sp = sub; sp < p.nsplit; sp += 8) {
+          const int64_t pr = base + (int64_t)sp * p.Mpad;
+          const float ms = p.part_m[pr];
+          l += ms == neg_inf() ? 0.f : exp2f_fast(ms - mx) * p.part_l[pr];
+        }
+#pragma unroll
+        for (int w = 1; w < 8; w <<= 1) l += __shfl_xor(l, w);
+        if (sub == 0) lse[v] = l > 0.f ? mx + log2f_fast(l) : pos_inf();
+      } else if (sub == 0) {
+        lse[v] = p.lse2[(int64_t)bh * p.M + pos];
+      }
+    }
+  }
+  __syncthreads();
+  const int key = 1024 * kb + 4 * tid;
+  if (key >= p.N) return;
+  const float* src = p.few + (int64_t)bhk * rows * p.few_pitch + key;
+  float acc[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 8
+  for (int r = 0; r < rows; ++r) {
+    const f32x4 x = *reinterpret_cast<const f32x4*>(src + (int64_t)r * p.few_pitch);
+    const float off = lse[r];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) acc[e] += exp2f_fast(fmaf(x[e], p.qk_scale, -off));
+  }
+  float* out = p.col + b * p.sc0 + hk * p.sc1;
+#pragma unroll
+  for (int e = 0; e < 4; ++e)
+    if (key + e < p.N) out[(int64_t)(key + e) * p.sc2] = acc[e];
+}
+
 template <class E, int D, int MODE, int NW, bool DROP, bool PACK, bool KS2 = false, bool ALN = true>
 hipError_t launch_fwd_t(const FwdParams& p, hipStream_t stream) {
   constexpr bool kCanSplit =
-      !KS2 && (MODE == kFwdPlain || MODE == kFwdPlainKeepBits || MODE == kFwdRowSum);
+      !KS2 && (MODE == kFwdPlain || MODE == kFwdPlainKeepBits || MODE == kFwdRowSum ||
+                MODE == kFwdFewRows);
   const int64_t nsplit = kCanSplit ? p.nsplit : 1;
   const dim3 grid((unsigned)((int64_t)p.nrb * (p.B * p.H / p.pack) * nsplit)), block(NW * 64);
   hipLaunchKernelGGL((fwd_kernel<E, D, MODE, NW, DROP, PACK, KS2, ALN>), grid, block, 0, stream, p);
   if constexpr (kCanSplit) {
-    if (p.nsplit > 1 && p.M > 0) {
+    // (kFwdFewRows with kept scores: launch_few_cols merges the splits.)
+    if (p.nsplit > 1 && p.M > 0 && !(MODE == kFwdFewRows && p.few != nullptr)) {
       const int64_t nblk = (p.M + 2048 / D - 1) / (2048 / D);
-      constexpr int CM = MODE == kFwdPlainKeepBits ? kFwdPlain : MODE;
+      constexpr int CM = MODE == kFwdRowSum ? kFwdRowSum : kFwdPlain;
       hipLaunchKernelGGL((fwd_combine_kernel<E, D, CM>),
                          dim3((unsigned)(nblk * p.B * p.H)), dim3(256), 0, stream, p);
     }

@@ -9,6 +9,7 @@ hipError_t launch_fwd_scores(const FwdParams& p, int dtype, int d, hipStream_t s
 hipError_t launch_fwd_scores_unaligned(const FwdParams& p, int dtype, int d, hipStream_t s);
 hipError_t launch_fwd_region(const FwdParams& p, int dtype, int d, hipStream_t s);
 hipError_t launch_fwd_key_split(const FwdParams& p, int mode, int dtype, int d, hipStream_t s);
+hipError_t launch_fwd_few(const FwdParams& p, int dtype, int d, hipStream_t s);
 hipError_t launch_fwd_dropout(const FwdParams& p, int mode, int dtype, int d, hipStream_t s);
 hipError_t launch_fwd_packed(const FwdParams& p, int mode, int dtype, int d, hipStream_t s);
 hipError_t launch_fwd_scores_packed(const FwdParams& p, int dtype, int d, hipStream_t s);
@@ -22,10 +23,11 @@ hipError_t launch_fwd(const FwdParams& p, int mode, int dtype, int d, hipStream_
   if (p.bm != kFwdRows) {
     if (mode == kFwdScores
             ? p.dropout || p.pack != 1 || (p.bm != kFwdRows / 2 && p.bm != kFwdRows / 4)
-            : mode == kFwdRegion || p.bm != kFwdRows / 2 || p.nsplit != 1)
+            : mode == kFwdRegion || mode == kFwdFewRows || p.bm != kFwdRows / 2 || p.nsplit != 1)
       return hipErrorInvalidValue;
     if (mode != kFwdScores && !p.dropout) return launch_fwd_key_split(p, mode, dtype, d, s);
   }
+  if (mode == kFwdFewRows) return launch_fwd_few(p, dtype, d, s);
   if (mode == kFwdScores && !p.scores_aligned) {
     if (p.pack > 1 && p.dropout) return hipErrorInvalidValue;
     return launch_fwd_scores_unaligned(p, dtype, d, s);

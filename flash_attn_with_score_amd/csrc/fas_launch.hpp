@@ -10,6 +10,11 @@ namespace fas {
 
 // Forward pass (fas_fwd.hpp); mode is a FwdMode, dtype 0 = fp16, 1 = bf16.
 hipError_t launch_fwd(const FwdParams& p, int mode, int dtype, int d, hipStream_t s);
+// After a kFwdFewRows pass: merges its key splits (or takes its lse2) and sums
+// the softmax weights of the kept scores per key.
+hipError_t launch_few_cols(const FwdParams& p, int dtype, int d, hipStream_t s);
+// Most query rows per KV head of kFwdFewRows: one wave's.
+constexpr int kFwdFewMax = 32;
 // Query rows per forward workgroup (8 wave64s x 32 rows).
 constexpr int kFwdRows = 256;
 

@@ -11,7 +11,8 @@ enum FwdMode : int {
   kFwdScores = 1,  // + (B,H,M,N) scaled scores, masked -> 0
   kFwdRowSum = 2,  // + (B,H,M) row sums of scaled scores
   kFwdRegion = 3,  // + fp32 raw scores of rows >= split, keys < split
-  kFwdPlainKeepBits = 4  // kFwdPlain with dropout, storing the keep decisions (drop_bits)
+  kFwdPlainKeepBits = 4,  // kFwdPlain with dropout, storing the keep decisions (drop_bits)
+  kFwdFewRows = 5  // kFwdPlain, at most 32 query rows per KV head: + the scores of every key
 };
 
 // Dropout of the attention weights with the reference's random stream:
@@ -105,6 +106,14 @@ struct FwdParams {
   float* part_m;     // (B*H, nsplit, Mpad) base-2 exponent offset, -inf if none
   float* part_l;     // (B*H, nsplit, Mpad) sum of the weights
   float* part_r;     // (B*H, nsplit, Mpad) raw row sums (kFwdRowSum)
+  // kFwdFewRows: the raw fp32 scores, row ((b*Hk + hk) * G*M + v) of virtual
+  // row v at pitch few_pitch (a multiple of 64), masked -inf; or, when few is
+  // null, the score matrix (scores).  col: (B, Hk, N) strided sums of the
+  // softmax weights over the G*M rows (launch_few_cols).
+  float* few;
+  int few_pitch;
+  float* col;
+  int64_t sc0, sc1, sc2;
   float sm_scale;    // |sm_scale|
   float qk_scale;    // |sm_scale| * log2(e)
   // Words workgroup 0 sets to zero before anything else: the tickets of the

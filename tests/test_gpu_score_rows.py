@@ -36,8 +36,11 @@ CASES = [
     (1, 8, 2, 90, 131, 64, True, 0, 0),       # four packed heads
     (1, 7, 1, 66, 129, 64, True, 4, 2),       # seven heads, unpacked writer
     (1, 2, 2, 1, 7, 64, True, 0, 1),          # less than one 16-byte unit
-    (1, 2, 2, 7, 2049, 64, True, 0, 0),       # key split, resident-Q scores
-    (2, 4, 2, 3, 4100, 128, True, 1, 0),      # the same over two packed heads
+    (1, 2, 2, 40, 2049, 64, True, 0, 0),      # key split, resident-Q scores
+    (2, 4, 2, 20, 4100, 128, True, 1, 0),     # the same over two packed heads
+    (1, 2, 2, 7, 2049, 64, True, 0, 1),       # few query rows: scores from the forward
+    (2, 4, 2, 16, 4100, 128, True, 1, 0),     # the same, 32 rows of two packed heads
+    (1, 3, 1, 1, 3007, 32, False, 0, 0),
     (1, 2, 2, 700, 3001, 32, True, 0, 0),     # key split, K-resident scores
 ]
 
