@@ -252,8 +252,8 @@ __device__ __forceinline__ int64_t* region_rows() {
 // PACK: GQA packing (p.pack query heads per workgroup, per-lane heads and
 // positions); without it the workgroup's rows are one head's and every
 // per-lane head offset folds away at compile time.
-// Two waves per SIMD, except for the 4-wave score writer (64-row blocks),
-// whose LDS (one workgroup per CU) allows one.
+// The 4-wave score writer (64-row blocks) runs one wave per SIMD (its LDS:
+// one workgroup per CU), the others two, or four (fwd_waves).
 // KS2 (unpacked score writer): row blocks of 32 * NW / 2 rows whose key
 // range is split between the wave pairs: loader wave i takes the even key
 // tiles and storer wave NW/2 + i the odd ones of the same 32 rows, so a step
@@ -270,8 +270,20 @@ __device__ __forceinline__ int64_t* region_rows() {
 //    storers, which store both tiles of the step during O += P V.
 // ALN (score writer): whether the score rows start on 64-byte boundaries
 // (store_score16).
+// Waves per SIMD (two workgroups a CU for four): up to D = 32 the step is the
+// exponentials and its waits, which a second workgroup fills (row sum B2 H16/8
+// S8568 D32 causal 283 -> 229 us, B1 H32 S4096 D16 72 -> 59); at D = 64 four
+// waves fit 128 registers too, but the VALU is busy with two (B1 H28/4 S4096
+// 81 -> 88 us, B2 H12 S8680 291 -> 283).
+constexpr int fwd_waves(int d, int mode, int nw, bool drop) {
+  return nw == 4 ? 1 : d <= 32 && mode != kFwdScores && mode != kFwdRegion && !drop ? 4 : 2;
+}
+constexpr int fwd_waves_max(int d, int mode, int nw, bool drop) {
+  return nw == 4 ? 2 : fwd_waves(d, mode, nw, drop);
+}
 template <class E, int D, int MODE, int NW, bool DROP, bool PACK, bool KS2 = false, bool ALN = true>
-__global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(NW == 4 ? 1 : 2, 2)))
+__global__ __launch_bounds__(NW * 64)
+__attribute__((amdgpu_waves_per_eu(fwd_waves(D, MODE, NW, DROP), fwd_waves_max(D, MODE, NW, DROP))))
 void fwd_kernel(const FwdParams p) {
   static_assert(MODE != kFwdScores || NW == 8 || NW == 4, "the score writer uses 4 or 8 waves");
   static_assert(!KS2 || !(MODE == kFwdScores && (DROP || PACK)),
@@ -279,6 +291,7 @@ void fwd_kernel(const FwdParams p) {
   static_assert(!KS2 || (MODE != kFwdRegion && MODE != kFwdFewRows),
                 "modes with key-split instances");
   static_assert(ALN || MODE == kFwdScores, "only the score writer has unaligned rows");
+  constexpr bool kTight = fwd_waves(D, MODE, NW, DROP) == 4;  // 128 registers
   constexpr int NH = NW / 2;  // score writer: loader waves [0, NH), storer waves [NH, NW)
   const int pack = PACK ? p.pack : 1;
   constexpr int KS = D / 16;               // MFMA k-steps over the head dim
@@ -347,6 +360,13 @@ void fwd_kernel(const FwdParams p) {
     if constexpr (kCanSplit) {
       split = bid % p.nsplit;
       bid /= p.nsplit;
+    }
+    if constexpr (kTight) {
+      // Two workgroups share a CU: with at most two for each, the second ones
+      // (8 XCDs x 32 CUs on) go shortest first beside the longest.
+      const int per = (p.nrb * (p.B * p.H / pack)) >> 3, s = bid >> 3;
+      if (p.causal && per > 32 && per <= 64 && s >= 32 && s < per)
+        bid = ((32 + per - 1 - s) << 3) | (bid & 7);
     }
     map_block(bid, p.nrb, p.B * p.H / pack, p.causal != 0, rb, grp);
   }
@@ -766,7 +786,18 @@ void fwd_kernel(const FwdParams p) {
         if (!ok) s[kb][r] = neg_inf();
       }
   };
+  const VtOff vto = vt_offsets<D>(lane);
   auto pv_mma = [&](const u32x4 (&pb)[4], const uint16_t* vt) __attribute__((always_inline)) {
+    if constexpr (kTight) {
+      VtOff o = vto;
+      opaque(o);
+#pragma unroll
+      for (int db = 0; db < DB; ++db)
+#pragma unroll
+        for (int cs = 0; cs < 4; ++cs)
+          oacc[db] = E::mma(lds_vt_operand<D>(vt, o, db, cs), pb[cs], oacc[db]);
+      return;
+    }
 #pragma unroll
     for (int db = 0; db < DB; ++db)
 #pragma unroll
@@ -890,7 +921,7 @@ void fwd_kernel(const FwdParams p) {
             sched_score_tile<KS, 0>();
           }
         } else {
-          score_tile(kt, s, tw, std::integral_constant<bool, kSplit>{});
+          score_tile(kt, s, tw, std::integral_constant<bool, kSplit || kTight>{});
           sched_score_tile<KS, 0>();
         }
         if (masked) apply_mask(s, k0);
