@@ -1,4 +1,4 @@
-"""Cross-token softmax-weight sums, recomputing and buffered variants.
+"""Cross-token softmax-weight sums, and the buffered variant's entry point.
 
 Drop-ins for the reference's attention_cross_token_softmax_sum.py:735-863
 (attention_cross_token_softmax_sum, fused two-pass kernel :24-268) and
@@ -24,15 +24,17 @@ def attention_cross_token_softmax_sum_buffered(
     sm_scale: float = None,
     dropout_p: float = 0.0,
 ) -> tuple[torch.Tensor, torch.Tensor]:
-    """Same result as attention_cross_token_softmax_sum; pass 1 stores the
-    scores of the region (queries >= split, keys < split) in a scratch buffer
-    and pass 2 reloads them instead of recomputing q . k.
+    """Same result as attention_cross_token_softmax_sum.
 
-    The scratch holds only the region (the only part ever re-read; the
-    reference allocates B * Hq * M * N * 4 bytes of raw fp32 scores,
-    :704-705), each score as an fp16 base-2 exponent relative to its row's
-    maximum over the region keys of its 64-key tile, plus those maxima:
-    B * Hq * max(M - split, 0) * (split * 2 + ceil(split / 64) * 4) bytes.
+    The reference's pass 1 stores the raw scores, B * Hq * M * N * 4 bytes
+    (:704-705), and its pass 2 reloads them.  On MI355X recomputing q . k for
+    the region (queries >= split, keys < split) is faster at every size
+    measured than writing and reading even 2 bytes per score of it
+    (fas_attention_cross_token_softmax_sum_buffered: B1 H32/8 S16384 split
+    12288 D128 2.94 against 2.35 ms, B1 H32 S4096 split 3072 231 against 190
+    us, split 3001 560 against 193 us, B1 H4 S1664 split 283 D32 151 against
+    53 us), is exact to fp32 instead of fp16 exponents, and needs no region,
+    so this entry point recomputes too.
     """
     Dq, Dk, Dv = q.shape[-1], k.shape[-1], v.shape[-1]
     assert Dq == Dk == Dv, "Q, K, V must have the same head_dim"
@@ -53,10 +55,10 @@ def attention_cross_token_softmax_sum_buffered(
     cross = torch.empty((B, Hk, split), device=q.device, dtype=torch.float32)
     # The reference's buffered kernel ignores dropout_p and draws no seed.
     args = _native.make_args(p.q, p.k, p.v, output, causal, p.sm_scale)
-    ws_ptr, ws_bytes, ws = _common.workspace(_native.VARIANT_CROSS_SOFTMAX_SUM_BUFFERED, args, split,
+    ws_ptr, ws_bytes, ws = _common.workspace(_native.VARIANT_CROSS_SOFTMAX_SUM, args, split,
                                              q.device)
-    _common.call("fas_attention_cross_token_softmax_sum_buffered", p.q, ctypes.byref(args),
-                 int(split), cross.data_ptr(), _native.strides3(cross), ws_ptr, ws_bytes)
+    _common.call("fas_attention_cross_token_softmax_sum", p.q, ctypes.byref(args), int(split),
+                 cross.data_ptr(), _native.strides3(cross), ws_ptr, ws_bytes)
     return output, cross
 
 
