@@ -344,7 +344,11 @@ struct ColPlan {
   int64_t nunits = 0, ngroups = 0;
 };
 constexpr int64_t kCus = 256;  // MI355X compute units
-ColPlan col_plan(const Problem& pr, bool buffered, int64_t ncols, bool fold_heads) {
+// Where that leaves CUs idle, the recomputing pass also splits its row steps
+// (128 rows of one head), to pieces of at least 2 of them: cost = rounds x
+// (steps of a workgroup + 3 for its K loads and the fold).
+ColPlan col_plan(const Problem& pr, bool buffered, int64_t ncols, bool fold_heads,
+                 int64_t row_lo, bool split_rows) {
   ColPlan c;
   c.fold = fold_heads ? pr.G : 1;
   c.ngroups = (int64_t)pr.B * (pr.H / c.fold);
@@ -363,6 +367,30 @@ ColPlan col_plan(const Problem& pr, bool buffered, int64_t ncols, bool fold_head
     if (cost < best) {
       best = cost;
       c.nsplit = ns;
+    }
+  }
+  if (buffered || !fold_heads || !split_rows) return c;
+  // Steps of a unit's longest pair of blocks over the fold's heads.
+  auto steps = [&](int64_t kb) {
+    int64_t lo = row_lo;
+    if (pr.causal) lo = std::max<int64_t>(lo, 256 * kb - ((int64_t)pr.N - pr.M));
+    return std::max<int64_t>(0, (pr.M + 127) / 128 - std::max<int64_t>(0, lo) / 128);
+  };
+  const int64_t nkb = (ncols + 255) / 256;
+  if (nkb == 0) return c;
+  const int64_t total = c.fold * (steps(0) + (nkb > 1 ? steps(nkb - 1) : 0));
+  const int64_t wgs = c.nunits * c.ngroups;
+  const int heads = c.nsplit;
+  auto cost_of = [&](int64_t ns) {
+    return ((wgs * ns + slots - 1) / slots) * ((total + ns - 1) / ns + 3);
+  };
+  best = cost_of(heads);
+  for (int m = 2; m <= 8; ++m) {
+    const int64_t ns = (int64_t)heads * m;
+    if (c.fold * steps(0) < 2 * ns) break;
+    if (cost_of(ns) < best) {
+      best = cost_of(ns);
+      c.nsplit = (int)ns;
     }
   }
   return c;
@@ -690,7 +718,12 @@ Workspace layout(int variant, const Problem& pr, int64_t split, size_t budget = 
         off += bytes;
       }
     }
-    w.cp = col_plan(pr, variant == FAS_VARIANT_CROSS_SOFTMAX_SUM_BUFFERED, ncols, true);
+    const bool buffered = variant == FAS_VARIANT_CROSS_SOFTMAX_SUM_BUFFERED;
+    const int64_t row_lo = variant == FAS_VARIANT_SOFTMAX_COL_SUM ? 0 : split;
+    w.cp = col_plan(pr, buffered, ncols, true, row_lo, true);
+    // Without room for that many partials, the heads' split alone.
+    if (off + (size_t)w.cp.ngroups * (w.cp.nsplit * ncols + w.cp.nunits) * 4 + 512 > budget)
+      w.cp = col_plan(pr, buffered, ncols, true, row_lo, false);
     if (w.has_few) w.cp.nsplit = 1;
     if (w.cp.nsplit > 1) {
       // The splits' column sums and one ticket per (output group, unit).

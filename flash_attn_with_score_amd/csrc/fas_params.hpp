@@ -145,9 +145,10 @@ struct ColsmParams {
   int B, H, G, M, N;
   // Head folding: output column group og = b * (H / fold) + ho sums the
   // query heads ho*fold .. ho*fold + fold - 1 (fold = G: the column sums per
-  // KV head; fold = 1: per query head, total_attention).  The fold's heads
-  // are dealt to nsplit workgroups per key block (pair), split s taking
-  // heads s, s + nsplit, ...; with nsplit > 1 each writes its column sums to
+  // KV head; fold = 1: per query head, total_attention).  The fold's rows are
+  // dealt to nsplit workgroups per key block (pair): equal runs of its steps
+  // of 128 rows in head order (colsm64_kernel), or heads s, s + nsplit, ...
+  // (the buffered pass); with nsplit > 1 each writes its column sums to
   // part[(og * nsplit + s) * ncols + key] and bumps ticket[og * nunits +
   // unit] (unit = the key block or pair), and the workgroup that brings the
   // ticket to nsplit adds the nsplit partials in split order into out.

@@ -11,8 +11,8 @@
 // deterministic.
 // GQA groups are folded inside the pass: a workgroup walks the query heads
 // of its KV head with its keys resident, or, when that would leave CUs idle,
-// shares them with other workgroups and the last one to finish adds their
-// column sums in a fixed order.
+// shares their rows with other workgroups and the last one to finish adds
+// their column sums in a fixed order.
 //
 // Raw-score column sums (attention_with_col_sum.py:186-191,
 // attention_with_col_sum_sequential.py:177-182,
@@ -180,8 +180,6 @@ void colsm64_kernel(const ColsmParams p) {
   const int b = item.og / hout, ho = item.og - b * hout;
   const int hfirst = ho * p.fold;   // first query head of the output group
   const int hk = hfirst / p.G;
-  // Heads of this split: hfirst + j, j = sp, sp + nsplit, ... < fold.
-  const int nheads = (p.fold - item.sp + p.nsplit - 1) / p.nsplit;
   const int kbb = p.nkb - 1 - pb;
 
   const __amdgpu_buffer_rsrc_t rk = make_rsrc(p.k + b * p.sk0 + hk * p.sk1, p.k_bytes);
@@ -260,7 +258,9 @@ void colsm64_kernel(const ColsmParams p) {
     if (p.causal) rstart = max(rstart, kb * BK - p.causal_off);
     const int t0 = max(0, rstart) / TQ;
     const int nt = t1 > t0 ? t1 - t0 : 0;
-    const int nsteps = nheads * nt;  // (head, step) pairs, head-major
+    // This split's share of the block's (head, step) pairs, head-major.
+    const int first = (int)((int64_t)p.fold * nt * item.sp / p.nsplit);
+    const int nsteps = (int)((int64_t)p.fold * nt * (item.sp + 1) / p.nsplit) - first;
 
     float colacc[2] = {0.f, 0.f};
     // Keep words of step t of head h (DROP == 2): block (qb, j) is rows
@@ -283,11 +283,15 @@ void colsm64_kernel(const ColsmParams p) {
       }
     };
     // The step being computed (head ch, row step ct) and the one after it.
-    int ch = hfirst + item.sp, ct = t0;
+    int ch = hfirst, ct = t0;
+    if (nsteps > 0) {
+      ch += first / nt;
+      ct += first % nt;
+    }
     auto advance = [&](int& h, int& t) __attribute__((always_inline)) {
       if (++t == t1) {
         t = t0;
-        h += p.nsplit;
+        ++h;
       }
     };
     if (nsteps > 0) {
