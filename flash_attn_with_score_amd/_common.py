@@ -32,7 +32,8 @@ def _rows_aligned(x: torch.Tensor) -> bool:
 
 
 def as_kernel_operand(x: torch.Tensor) -> torch.Tensor:
-    if x.stride(-1) == 1 and _rows_aligned(x):
+    s = x.stride()
+    if len(s) == 4 and s[3] == 1 and not ((x.data_ptr() & 15) | ((s[0] | s[1] | s[2]) & 7)):
         return x
     x = maybe_contiguous(x)
     return x if _rows_aligned(x) else x.contiguous()
@@ -91,7 +92,11 @@ def finish_problem(q, k, v, sm_scale) -> Problem:
 
 
 def new_output(q: torch.Tensor) -> torch.Tensor:
+    """An output like q, a kernel operand: with q's strides (empty_like of a
+    dense q) it is one wherever q is, the allocator's addresses being aligned."""
     o = torch.empty_like(q)
+    if o.stride() == q.stride() and not o.data_ptr() & 15:
+        return o
     return o if _rows_aligned(o) and o.stride(-1) == 1 else torch.empty(
         q.shape, dtype=q.dtype, device=q.device)
 
@@ -103,19 +108,24 @@ def _raw_stream(index: int) -> int:
 # torch's current stream of a device as a raw handle without building a
 # Stream object (the call costs ~0.3 us instead of several).
 _current_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", _raw_stream)
+_current_device = getattr(torch._C, "_cuda_getDevice", torch.cuda.current_device)
 
 
 def call(fn_name: str, q: torch.Tensor, *args) -> None:
-    """Invokes one C entry point on q's device and torch's current stream."""
-    lib = _native.load()
-    fn = getattr(lib, fn_name)
+    """Invokes one C entry point (_native.fast: records as bytes) on q's device
+    and torch's current stream."""
+    fn = _native.fast(fn_name)
     index = q.device.index
-    if index == torch.cuda.current_device():
+    if index == _current_device():
         rc = fn(*args, _current_raw_stream(index))
     else:
         with torch.cuda.device(index):
             rc = fn(*args, _current_raw_stream(index))
-    _native.check(lib, rc, fn_name)
+    if rc:
+        _native.check(_native.load(), rc, fn_name)
+
+
+_SIZE_MAX = (1 << 64) - 1
 
 
 def workspace(variant: int, args, split: int, device,
@@ -124,12 +134,12 @@ def workspace(variant: int, args, split: int, device,
     allocator, 256-byte aligned) and returns (pointer, bytes, tensor); with
     `limit`, a workspace larger than that is not allocated (pointer 0, no
     tensor) and the caller takes its route without it."""
-    import ctypes
-
-    lib = _native.load()
-    nbytes = lib.fas_workspace_bytes(variant, ctypes.byref(args), int(split))
-    if nbytes == ctypes.c_size_t(-1).value:
-        raise RuntimeError(f"fas_workspace_bytes: {_native.last_error(lib) or 'invalid request'}")
+    if type(args) is not bytes:  # an AttnArgs
+        args = bytes(args)
+    nbytes = _native.fast("fas_workspace_bytes")(variant, args, int(split))
+    if nbytes == _SIZE_MAX:
+        raise RuntimeError(
+            f"fas_workspace_bytes: {_native.last_error(_native.load()) or 'invalid request'}")
     if nbytes == 0 or (limit is not None and nbytes > limit):
         return 0, nbytes, None
     buf = torch.empty(nbytes + 256, dtype=torch.uint8, device=device)

@@ -89,6 +89,12 @@ def make_args(q, k, v, o, causal: bool, sm_scale: float, dropout=None,
               keep_bits: int | None = 0) -> AttnArgs:
     """dropout: None, or (dropout_p, seed, offset) of the reference's stream;
     keep_bits: device address of the forward's keep-bit buffer, or 0 (None: 0)."""
+    return AttnArgs.from_buffer_copy(pack_args(q, k, v, o, causal, sm_scale, dropout, keep_bits))
+
+
+def pack_args(q, k, v, o, causal: bool, sm_scale: float, dropout=None,
+              keep_bits: int | None = 0) -> bytes:
+    """The same record as bytes, which the entry points of fast() take as they are."""
     B, H, M, D = q.shape
     if dropout is None:
         dp, seed, offset = 0.0, 0, 0
@@ -96,12 +102,21 @@ def make_args(q, k, v, o, causal: bool, sm_scale: float, dropout=None,
         dp = float(dropout[0])
         seed = int(dropout[1]) & 0xFFFFFFFFFFFFFFFF
         offset = int(dropout[2]) & 0xFFFFFFFFFFFFFFFF
-    return AttnArgs.from_buffer_copy(_ARGS_PACK.pack(
+    ks = k.shape
+    return _ARGS_PACK.pack(
         DTYPE_CODES[q.dtype], 1 if causal else 0, float(sm_scale), 0,
-        B, H, k.shape[1], M, k.shape[2], D,
+        B, H, ks[1], M, ks[2], D,
         q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(),
         *q.stride(), *k.stride(), *v.stride(), *o.stride(),
-        dp, 0, seed, offset, keep_bits or 0))
+        dp, 0, seed, offset, keep_bits or 0)
+
+
+_STRIDES = (None, None, None, struct.Struct("<3q").pack, struct.Struct("<4q").pack)
+
+
+def pack_strides(t: torch.Tensor) -> bytes:
+    s = t.stride()
+    return _STRIDES[len(s)](*s)
 
 
 _P = ctypes.POINTER
@@ -151,6 +166,7 @@ def library_path() -> Path:
 
 _lock = threading.Lock()
 _lib = None
+_fast: dict = {}
 
 
 def load() -> ctypes.CDLL:
@@ -175,8 +191,24 @@ def load() -> ctypes.CDLL:
         version = lib.fas_abi_version()
         if version != ABI_VERSION:
             raise RuntimeError(f"libfas.so ABI version {version}, expected {ABI_VERSION}")
+        # The same entry points taking their records as bytes: no ctypes
+        # structure or array is built per call.
+        records = ctypes.CDLL(str(path))
+        swap = {_P(AttnArgs): ctypes.c_char_p, _I64x4: ctypes.c_char_p, _I64x3: ctypes.c_char_p}
+        for name, (restype, argtypes) in _SIGNATURES.items():
+            fn = getattr(records, name)
+            fn.restype = restype
+            fn.argtypes = [swap.get(t, t) for t in argtypes]
+            _fast[name] = fn
         _lib = lib
         return lib
+
+
+def fast(name: str):
+    """The entry point that takes fas_attn_args and strides as bytes."""
+    if _lib is None:
+        load()
+    return _fast[name]
 
 
 def last_error(lib) -> str:

@@ -6,7 +6,6 @@ Drop-ins for the reference's attention_cross_token_softmax_sum.py:735-863
 """
 from __future__ import annotations
 
-import ctypes
 
 import torch
 
@@ -54,11 +53,11 @@ def attention_cross_token_softmax_sum_buffered(
     output = _common.new_output(p.q)
     cross = torch.empty((B, Hk, split), device=q.device, dtype=torch.float32)
     # The reference's buffered kernel ignores dropout_p and draws no seed.
-    args = _native.make_args(p.q, p.k, p.v, output, causal, p.sm_scale)
+    args = _native.pack_args(p.q, p.k, p.v, output, causal, p.sm_scale)
     ws_ptr, ws_bytes, ws = _common.workspace(_native.VARIANT_CROSS_SOFTMAX_SUM, args, split,
                                              q.device)
-    _common.call("fas_attention_cross_token_softmax_sum", p.q, ctypes.byref(args), int(split),
-                 cross.data_ptr(), _native.strides3(cross), ws_ptr, ws_bytes)
+    _common.call("fas_attention_cross_token_softmax_sum", p.q, args, int(split),
+                 cross.data_ptr(), _native.pack_strides(cross), ws_ptr, ws_bytes)
     return output, cross
 
 
@@ -91,10 +90,10 @@ def attention_cross_token_softmax_sum(
     p = _common.finish_problem(q, k, v, sm_scale)
     output = _common.new_output(p.q)
     cross = torch.empty((B, Hk, split), device=q.device, dtype=torch.float32)
-    args = _native.make_args(p.q, p.k, p.v, output, causal, p.sm_scale,
+    args = _native.pack_args(p.q, p.k, p.v, output, causal, p.sm_scale,
                              _common.draw_dropout(p.q, p.k, dropout_p))
     ws_ptr, ws_bytes, ws = _common.workspace(_native.VARIANT_CROSS_SOFTMAX_SUM, args, split,
                                              q.device)
-    _common.call("fas_attention_cross_token_softmax_sum", p.q, ctypes.byref(args), int(split),
-                 cross.data_ptr(), _native.strides3(cross), ws_ptr, ws_bytes)
+    _common.call("fas_attention_cross_token_softmax_sum", p.q, args, int(split),
+                 cross.data_ptr(), _native.pack_strides(cross), ws_ptr, ws_bytes)
     return output, cross

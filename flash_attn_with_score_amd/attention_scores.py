@@ -7,7 +7,6 @@ the scores-only gfx950 kernel through fas_attention_scores.
 """
 from __future__ import annotations
 
-import ctypes
 import math
 
 import torch
@@ -38,7 +37,7 @@ def compute_attention_scores(
     q, k = _common.as_kernel_operand(q), _common.as_kernel_operand(k)
     scores = torch.empty((B, H, M, N), dtype=q.dtype, device=q.device)
     # causal is accepted and ignored, as in the reference (attention_scores.py:166).
-    args = _native.make_args(q, k, k, q, False, float(sm_scale))
-    _common.call("fas_attention_scores", q, ctypes.byref(args), scores.data_ptr(),
-                 _native.strides4(scores))
+    args = _native.pack_args(q, k, k, q, False, float(sm_scale))
+    _common.call("fas_attention_scores", q, args, scores.data_ptr(),
+                 _native.pack_strides(scores))
     return scores

@@ -6,7 +6,6 @@ Drop-in for the reference's attention_with_col_sum_sequential.py:214-341
 """
 from __future__ import annotations
 
-import ctypes
 
 import torch
 
@@ -37,9 +36,9 @@ def attention_with_col_sum_sequential(
     p = _common.finish_problem(q, k, v, sm_scale)
     o = _common.new_output(p.q)
     col_sum = torch.empty((B, Hk, N), device=q.device, dtype=torch.float32)
-    args = _native.make_args(p.q, p.k, p.v, o, causal, p.sm_scale,
+    args = _native.pack_args(p.q, p.k, p.v, o, causal, p.sm_scale,
                              _common.draw_dropout(p.q, p.k, dropout_p))
     ws_ptr, ws_bytes, ws = _common.workspace(_native.VARIANT_COL_SUM_SEQUENTIAL, args, 0, q.device)
-    _common.call("fas_attention_with_col_sum_sequential", p.q, ctypes.byref(args), col_sum.data_ptr(),
-                 _native.strides3(col_sum), ws_ptr, ws_bytes)
+    _common.call("fas_attention_with_col_sum_sequential", p.q, args, col_sum.data_ptr(),
+                 _native.pack_strides(col_sum), ws_ptr, ws_bytes)
     return o, col_sum

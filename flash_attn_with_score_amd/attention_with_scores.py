@@ -7,7 +7,6 @@ torch.empty rather than zero-filled as the reference does (:284).
 """
 from __future__ import annotations
 
-import ctypes
 
 import torch
 
@@ -42,9 +41,9 @@ def attention_with_scores(
     p = _common.finish_problem(q, k, v, sm_scale)
     o = _common.new_output(p.q)
     scores = torch.empty((B, H, M, N), device=q.device, dtype=q.dtype)
-    args = _native.make_args(p.q, p.k, p.v, o, causal, p.sm_scale,
+    args = _native.pack_args(p.q, p.k, p.v, o, causal, p.sm_scale,
                              _common.draw_dropout(p.q, p.k, dropout_p))
     ws_ptr, ws_bytes, ws = _common.workspace(_native.VARIANT_SCORES, args, 0, q.device)
-    _common.call("fas_attention_with_scores", p.q, ctypes.byref(args), scores.data_ptr(),
-                 _native.strides4(scores), ws_ptr, ws_bytes)
+    _common.call("fas_attention_with_scores", p.q, args, scores.data_ptr(),
+                 _native.pack_strides(scores), ws_ptr, ws_bytes)
     return o, scores

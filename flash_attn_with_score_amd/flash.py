@@ -14,7 +14,6 @@ kernels for small grids and gives the same O and L.
 """
 from __future__ import annotations
 
-import ctypes
 import os
 
 import torch
@@ -60,23 +59,23 @@ def _forward(q, k, v, causal, sm_scale, want_total, dropout_p, keep=False):
     o = _common.new_output(p.q)
     L = torch.empty((p.B, p.H, p.M), device=q.device, dtype=torch.float32)
     drop = _common.draw_dropout(p.q, p.k, dropout_p)
-    args = _native.make_args(p.q, p.k, p.v, o, causal, p.sm_scale, drop)
+    args = _native.pack_args(p.q, p.k, p.v, o, causal, p.sm_scale, drop)
     kept = (0, None)
     if keep and drop is not None:
         kptr, _, kbuf = _common.workspace(_native.VARIANT_KEEP_BITS, args, 0, q.device,
                                           limit=KEEP_BITS_MAX_BYTES)
         if kbuf is not None:
-            args.keep_bits = kptr
+            args = _native.pack_args(p.q, p.k, p.v, o, causal, p.sm_scale, drop, kptr)
             kept = (kptr, kbuf)
     ws_ptr, ws_bytes, ws = _common.workspace(_native.VARIANT_ATTENTION_FORWARD, args, 0,
                                              q.device)
-    _common.call("fas_attention_forward", p.q, ctypes.byref(args), L.data_ptr(),
-                 _native.strides3(L), ws_ptr, ws_bytes)
+    _common.call("fas_attention_forward", p.q, args, L.data_ptr(),
+                 _native.pack_strides(L), ws_ptr, ws_bytes)
     tot = None
     if want_total:
         tot = torch.empty((p.B, p.H, p.N), device=q.device, dtype=torch.float32)
-        _common.call("fas_total_attention", p.q, ctypes.byref(args), L.data_ptr(),
-                     _native.strides3(L), tot.data_ptr(), _native.strides3(tot))
+        _common.call("fas_total_attention", p.q, args, L.data_ptr(),
+                     _native.pack_strides(L), tot.data_ptr(), _native.pack_strides(tot))
     return p, o, L, tot, drop, kept
 
 
@@ -122,7 +121,7 @@ class FlashAttention(torch.autograd.Function):
         dv = torch.empty((B, Hk, N, D), dtype=v.dtype, device=q.device)
         # The forward's (p, seed, offset): the same keep mask (flash.py:653-659),
         # read from the forward's bits when it kept them.
-        args = _native.make_args(q, k, v, o, ctx.causal, ctx.sm_scale, ctx.drop,
+        args = _native.pack_args(q, k, v, o, ctx.causal, ctx.sm_scale, ctx.drop,
                                  ctx.keep_ptr if ctx.keep_buf is not None else 0)
         try:
             ws_ptr, ws_bytes, ws = _common.workspace(_native.VARIANT_ATTENTION_BACKWARD, args, 0,
@@ -135,10 +134,10 @@ class FlashAttention(torch.autograd.Function):
             # Over the limit: the workspace without the stored dS (split != 0).
             ws_ptr, ws_bytes, ws = _common.workspace(_native.VARIANT_ATTENTION_BACKWARD, args,
                                                      1, q.device)
-        _common.call("fas_attention_backward", q, ctypes.byref(args), do.data_ptr(),
-                     _native.strides4(do), L.data_ptr(), _native.strides3(L), dq.data_ptr(),
-                     _native.strides4(dq), dk.data_ptr(), _native.strides4(dk), dv.data_ptr(),
-                     _native.strides4(dv), ws_ptr, ws_bytes)
+        _common.call("fas_attention_backward", q, args, do.data_ptr(),
+                     _native.pack_strides(do), L.data_ptr(), _native.pack_strides(L), dq.data_ptr(),
+                     _native.pack_strides(dq), dk.data_ptr(), _native.pack_strides(dk), dv.data_ptr(),
+                     _native.pack_strides(dv), ws_ptr, ws_bytes)
         return dq, dk, dv, None, None, None, None, None, None
 
 

@@ -9,7 +9,6 @@ head.
 """
 from __future__ import annotations
 
-import ctypes
 import math
 
 import torch
@@ -35,7 +34,7 @@ def total_attention(q, k, l, causal=False, sm_scale=None):
     assert l.dtype == torch.float32 and tuple(l.shape) == (B, H, M), "l must be (B, H, M) fp32"
     q, k = _common.as_kernel_operand(q), _common.as_kernel_operand(k)
     tot = torch.empty((B, H, N), dtype=torch.float32, device=q.device)
-    args = _native.make_args(q, k, k, q, causal, float(sm_scale))
-    _common.call("fas_total_attention", q, ctypes.byref(args), l.data_ptr(), _native.strides3(l),
-                 tot.data_ptr(), _native.strides3(tot))
+    args = _native.pack_args(q, k, k, q, causal, float(sm_scale))
+    _common.call("fas_total_attention", q, args, l.data_ptr(), _native.pack_strides(l),
+                 tot.data_ptr(), _native.pack_strides(tot))
     return tot
