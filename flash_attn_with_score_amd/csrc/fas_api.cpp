@@ -332,8 +332,8 @@ struct SplitPlan {
 // workgroup per (unit, split, output group), a unit being a mirror pair of
 // 256-key blocks (colsm64_kernel) or one key block (the buffered pass).
 // With fold heads per output column, nsplit workgroups share a unit's heads
-// (heads s, s + nsplit, ...) and fold their column sums through partials and
-// a ticket per unit; nsplit is the smallest of least cost, cost = rounds of
+// (equal runs of their steps; the buffered pass: heads s, s + nsplit, ...) and
+// fold their column sums through partials and a ticket per unit; nsplit is the smallest of least cost, cost = rounds of
 // `slots` concurrent workgroups x heads per workgroup, so a problem with few
 // output groups still fills the chip (B1 with 4 KV heads of 7 query heads:
 // 7 splits, 224 workgroups), and one that fills it walks all of a KV head's
@@ -1187,7 +1187,7 @@ static int attention_with_scores_impl(const fas_attn_args* a, void* scores, cons
        ((int64_t)(pw.pack - 1) * st[1] + (int64_t)(bm / pw.pack + 2) * st[2]) * 2 >= kMaxSliceBytes))
     pw.pack = 1;
   // One workgroup runs per CU, so with 256-row blocks in one round the
-  // longest row block sets the time.  Unpacked launches without dropout
+  // longest row block sets the time.  Launches without dropout
   // (whose instances have 256-row blocks only) then take 128- or 64-row
   // blocks whose key tiles are split between wave pairs (KS2): half or a
   // quarter of the rows, half the steps.  Measured (us, 256 / 128 / 64 rows):
@@ -1207,9 +1207,12 @@ static int attention_with_scores_impl(const fas_attn_args* a, void* scores, cons
   //    111; B1 H16 S3072 103.8 / 78.4);
   //  * else 256 rows (B1 H32 S2048 full 94.9 / 124.3 / 163.5; B2 H16 S1536 D64
   //    full 45.1 / 53.7 / 60.7).
+  // Grouped heads, which 256-row blocks pack, go one by one there too (packed /
+  // unpacked, causal D128: B1 H32/8 S1024 45.2 / 29.7, B1 H16/4 S4096 177 / 134,
+  // B1 H8/2 S4096 142 / 86; B1 H32/8 S3072, 256 rows: 145 / 172).
   const int64_t cus = device_cu_count();
   const int aligned = score_rows_aligned(scores, st, pr.N);
-  if (pw.pack == 1 && !(a->dropout_p > 0.f)) {
+  if (!(a->dropout_p > 0.f)) {
     const int64_t heads = (int64_t)pr.B * pr.H;
     const int64_t n256 = heads * ((pr.M + 255) / 256), n128 = heads * ((pr.M + 127) / 128),
                   n64 = heads * ((pr.M + 63) / 64);
@@ -1219,6 +1222,7 @@ static int attention_with_scores_impl(const fas_attn_args* a, void* scores, cons
     else if (n128 <= cus ||
              (n256 <= cus && pr.causal && pr.N >= 1024 && (n128 <= cus * 7 / 4 || pr.N >= 3072)))
       bm = 128;
+    if (bm != fas::kFwdRows) pw.pack = 1;
   }
   fas::FwdParams p = fwd_params(a, pw, false, bm);
   rescale_dropout(p, a);

@@ -786,23 +786,22 @@ void fwd_kernel(const FwdParams p) {
         if (!ok) s[kb][r] = neg_inf();
       }
   };
-  const VtOff vto = vt_offsets<D>(lane);
   auto pv_mma = [&](const u32x4 (&pb)[4], const uint16_t* vt) __attribute__((always_inline)) {
     if constexpr (kTight) {
-      VtOff o = vto;
+      VtOff o = vt_offsets<D>(lane);
       opaque(o);
 #pragma unroll
       for (int db = 0; db < DB; ++db)
 #pragma unroll
         for (int cs = 0; cs < 4; ++cs)
           oacc[db] = E::mma(lds_vt_operand<D>(vt, o, db, cs), pb[cs], oacc[db]);
-      return;
+    } else {
+#pragma unroll
+      for (int db = 0; db < DB; ++db)
+#pragma unroll
+        for (int cs = 0; cs < 4; ++cs)
+          oacc[db] = E::mma(lds_vt_operand<D>(vt, db, cs, lane), pb[cs], oacc[db]);
     }
-#pragma unroll
-    for (int db = 0; db < DB; ++db)
-#pragma unroll
-      for (int cs = 0; cs < 4; ++cs)
-        oacc[db] = E::mma(lds_vt_operand<D>(vt, db, cs, lane), pb[cs], oacc[db]);
   };
 
   if constexpr (kRegion) {

@@ -33,7 +33,8 @@ CASES = [
     (1, 64, 64, 520, 1031, 16, True, 0, 3),   # 128-row blocks, two rounds
     (1, 300, 300, 33, 67, 16, False, 0, 0),   # 256-row blocks
     (1, 300, 300, 70, 70, 32, True, 2, 5),    # 256-row blocks, causal zeros
-    (1, 8, 2, 90, 131, 64, True, 0, 0),       # four packed heads
+    (1, 8, 2, 90, 131, 64, True, 0, 0),       # grouped heads one by one
+    (40, 8, 2, 33, 67, 16, True, 0, 0),       # 256-row blocks of four packed heads
     (1, 7, 1, 66, 129, 64, True, 4, 2),       # seven heads, unpacked writer
     (1, 2, 2, 1, 7, 64, True, 0, 1),          # less than one 16-byte unit
     (1, 2, 2, 40, 2049, 64, True, 0, 0),      # key split, resident-Q scores
