@@ -13,6 +13,11 @@ from . import _common, _native
 
 __all__ = ["attention_cross_token_softmax_sum", "attention_cross_token_softmax_sum_buffered"]
 
+# Most query rows past the split for which the buffered variant keeps the
+# region's scores: a column pass of its own costs more than the little it
+# writes (B4 H4 S296 split 250 D128: 23.0 buffered, 24.2 us recomputed).
+BUFFERED_ROWS = 64
+
 
 def attention_cross_token_softmax_sum_buffered(
     q: torch.Tensor,
@@ -27,13 +32,13 @@ def attention_cross_token_softmax_sum_buffered(
 
     The reference's pass 1 stores the raw scores, B * Hq * M * N * 4 bytes
     (:704-705), and its pass 2 reloads them.  On MI355X recomputing q . k for
-    the region (queries >= split, keys < split) is faster at every size
-    measured than writing and reading even 2 bytes per score of it
+    the region (queries >= split, keys < split) is faster than writing and reading even 2 bytes per score of it
     (fas_attention_cross_token_softmax_sum_buffered: B1 H32/8 S16384 split
     12288 D128 2.94 against 2.35 ms, B1 H32 S4096 split 3072 231 against 190
     us, split 3001 560 against 193 us, B1 H4 S1664 split 283 D32 151 against
     53 us), is exact to fp32 instead of fp16 exponents, and needs no region,
-    so this entry point recomputes too.
+    so this entry point recomputes too, but for the few rows of
+    BUFFERED_ROWS.
     """
     Dq, Dk, Dv = q.shape[-1], k.shape[-1], v.shape[-1]
     assert Dq == Dk == Dv, "Q, K, V must have the same head_dim"
@@ -54,10 +59,12 @@ def attention_cross_token_softmax_sum_buffered(
     cross = torch.empty((B, Hk, split), device=q.device, dtype=torch.float32)
     # The reference's buffered kernel ignores dropout_p and draws no seed.
     args = _native.pack_args(p.q, p.k, p.v, output, causal, p.sm_scale)
-    ws_ptr, ws_bytes, ws = _common.workspace(_native.VARIANT_CROSS_SOFTMAX_SUM, args, split,
-                                             q.device)
-    _common.call("fas_attention_cross_token_softmax_sum", p.q, args, int(split),
-                 cross.data_ptr(), _native.pack_strides(cross), ws_ptr, ws_bytes)
+    variant, entry = _native.VARIANT_CROSS_SOFTMAX_SUM, "fas_attention_cross_token_softmax_sum"
+    if M - split <= BUFFERED_ROWS:
+        variant, entry = _native.VARIANT_CROSS_SOFTMAX_SUM_BUFFERED, entry + "_buffered"
+    ws_ptr, ws_bytes, ws = _common.workspace(variant, args, split, q.device)
+    _common.call(entry, p.q, args, int(split), cross.data_ptr(), _native.pack_strides(cross), ws_ptr,
+                 ws_bytes)
     return output, cross
 
 
