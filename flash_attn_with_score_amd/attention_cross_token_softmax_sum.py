@@ -13,10 +13,12 @@ from . import _common, _native
 
 __all__ = ["attention_cross_token_softmax_sum", "attention_cross_token_softmax_sum_buffered"]
 
-# Most query rows past the split for which the buffered variant keeps the
-# region's scores: a column pass of its own costs more than the little it
-# writes (B4 H4 S296 split 250 D128: 23.0 buffered, 24.2 us recomputed).
-BUFFERED_ROWS = 64
+# The buffered variant keeps the region's scores only for at most
+# BUFFERED_ROWS query rows past the split over at most BUFFERED_KEYS keys, where
+# a column pass of its own costs more than the little it writes (us, buffered /
+# recomputed, D128: B4 H4 S296 split 250 23.4 / 24.6, split 232 20.6 / 24.5; B1
+# H12 S704 split 640 34.3 / 32.0; B1 H32 S2048 split 2000 79.5 / 63.0).
+BUFFERED_ROWS, BUFFERED_KEYS = 64, 512
 
 
 def attention_cross_token_softmax_sum_buffered(
@@ -60,7 +62,7 @@ def attention_cross_token_softmax_sum_buffered(
     # The reference's buffered kernel ignores dropout_p and draws no seed.
     args = _native.pack_args(p.q, p.k, p.v, output, causal, p.sm_scale)
     variant, entry = _native.VARIANT_CROSS_SOFTMAX_SUM, "fas_attention_cross_token_softmax_sum"
-    if M - split <= BUFFERED_ROWS:
+    if M - split <= BUFFERED_ROWS and N <= BUFFERED_KEYS:
         variant, entry = _native.VARIANT_CROSS_SOFTMAX_SUM_BUFFERED, entry + "_buffered"
     ws_ptr, ws_bytes, ws = _common.workspace(variant, args, split, q.device)
     _common.call(entry, p.q, args, int(split), cross.data_ptr(), _native.pack_strides(cross), ws_ptr,
