@@ -1123,8 +1123,9 @@ static int run_scores(const char* fn, const fas_attn_args* a, const Problem& pr,
   // Up to 512 query rows: the resident-Q kernel, one workgroup per CU, each
   // walking two or more of its head's 512-key blocks.
   // Under GQA a workgroup takes the largest power-of-two share of a KV
-  // head's query heads whose rows fit (K loaded once for all of them), as
-  // long as its q and score offsets stay 31-bit.
+  // head's query heads, up to eight (the kernel's limit), whose rows fit (K
+  // loaded once for all of them), as long as its q and score offsets stay
+  // 31-bit.
   if (pr.M <= fas::kScoresResidentRows) {
     const int64_t nkb = (pr.N + fas::kScoresResidentKeys - 1) / fas::kScoresResidentKeys;
     int pshift = 0;
@@ -1135,7 +1136,7 @@ static int run_scores(const char* fn, const fas_attn_args* a, const Problem& pr,
                      2 <
                  fas::kScoresResidentBytes;
     };
-    while (fits(2 << pshift)) ++pshift;
+    while (pshift < 3 && fits(2 << pshift)) ++pshift;
     const int64_t groups = ((int64_t)pr.B * pr.H) >> pshift;
     const int64_t ngrp = std::min<int64_t>(nkb, (device_cu_count() + groups - 1) / groups);
     if (fits(1) && nkb >= 2 * ngrp) {

@@ -43,6 +43,7 @@ CASES = [
     (2, 4, 2, 16, 4100, 128, True, 1, 0),     # the same, 32 rows of two packed heads
     (1, 3, 1, 1, 3007, 32, False, 0, 0),
     (1, 2, 2, 700, 3001, 32, True, 0, 0),     # key split, K-resident scores
+    (64, 32, 1, 2, 2049, 16, True, 0, 0),     # 32 heads of a KV head, packed by eight
 ]
 
 

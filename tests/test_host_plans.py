@@ -1,0 +1,106 @@
+"""The launches that the C ABI's host code plans, without a GPU.
+
+fas_api.cpp is compiled with stand-ins for the kernel launchers
+(tests/plans/launch_log.cpp) that log each launch's mode, row blocks and
+splits.  Requests carry fake pointers that nothing dereferences.  Every call
+takes the workspace that fas_workspace_bytes asks for, as the launchers do.
+"""
+from __future__ import annotations
+
+import ctypes
+import os
+import subprocess
+
+import pytest
+
+from flash_attn_with_score_amd import _native
+from flash_attn_with_score_amd.csrc import build as fas_build
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+PTR = 0x1000000  # 256-byte aligned
+PLAIN, SCORES, ROWSUM, FEW = 0, 1, 2, 5  # FwdMode
+
+
+@pytest.fixture(scope="module")
+def lib(tmp_path_factory):
+    tmp = tmp_path_factory.mktemp("plans")
+    flags = ["-O1", "-std=c++17", "-fPIC", f"--offload-arch={fas_build.ARCH}",
+             f"-I{os.path.join(ROOT, 'include')}", f"-I{fas_build.CSRC}"]
+    objs = []
+    for src in (fas_build.CSRC / "fas_api.cpp", os.path.join(ROOT, "tests/plans/launch_log.cpp")):
+        objs.append(str(tmp / (os.path.basename(src) + ".o")))
+        subprocess.run([fas_build.hipcc(), "-x", "hip", *flags, "-c", str(src), "-o", objs[-1]],
+                       check=True, capture_output=True, text=True)
+    so = str(tmp / "plans.so")
+    subprocess.run([fas_build.hipcc(), "-shared", "-fPIC", f"--offload-arch={fas_build.ARCH}",
+                    *objs, "-o", so], check=True, capture_output=True, text=True)
+    lib = ctypes.CDLL(so)
+    for name, (restype, argtypes) in _native._SIGNATURES.items():
+        fn = getattr(lib, name)
+        fn.restype, fn.argtypes = restype, argtypes
+    lib.plan_log_take.restype = ctypes.c_char_p
+    return lib
+
+
+def make_args(B, Hq, Hk, M, N, D, causal=1, dropout=0.0, dtype=1):
+    a = _native.AttnArgs()
+    a.dtype, a.causal, a.sm_scale = dtype, causal, D ** -0.5
+    a.batch, a.heads_q, a.heads_k, a.seqlen_q, a.seqlen_k, a.head_dim = B, Hq, Hk, M, N, D
+    a.q = a.k = a.v = a.out = PTR
+    for name, H, L in (("q_stride", Hq, M), ("k_stride", Hk, N), ("v_stride", Hk, N),
+                       ("out_stride", Hq, M)):
+        setattr(a, name, _native._I64x4(H * L * D, L * D, D, 1))
+    a.dropout_p = dropout
+    return a
+
+
+def take(lib):
+    """The logged launches: [(name, {field: value})]."""
+    out = []
+    for line in lib.plan_log_take().decode().splitlines():
+        name, *fields = line.split()
+        out.append((name, {k: int(v) for k, v in (f.split("=") for f in fields)}))
+    return out
+
+
+def launches(lib, entry, a, split=0):
+    """Sends one request with the workspace it asks for; returns its launches."""
+    B, H, Hk, M, N = a.batch, a.heads_q, a.heads_k, a.seqlen_q, a.seqlen_k
+    q4, k4 = a.q_stride, a.k_stride
+    rows, keys = _native._I64x3(H * M, M, 1), _native._I64x3(Hk * N, N, 1)
+    s4 = _native._I64x4(H * M * N, M * N, N, 1)
+    variant = getattr(_native, "VARIANT_" + entry.upper())
+    nbytes = lib.fas_workspace_bytes(variant, ctypes.byref(a), split)
+    ws = (PTR, nbytes, None)
+    ref = ctypes.byref(a)
+    take(lib)
+    if entry == "scores":
+        rc = lib.fas_attention_with_scores(ref, PTR, s4, *ws)
+    elif entry == "row_sum":
+        rc = lib.fas_attention_with_row_sum(ref, PTR, rows, *ws)
+    elif entry == "softmax_col_sum":
+        rc = lib.fas_attention_with_softmax_col_sum(ref, PTR, keys, *ws)
+    elif entry == "cross_softmax_sum":
+        rc = lib.fas_attention_cross_token_softmax_sum(ref, split, PTR,
+                                                       _native._I64x3(Hk * split, split, 1), *ws)
+    elif entry == "attention_backward":
+        rc = lib.fas_attention_backward(ref, PTR, q4, PTR, rows, PTR, q4, PTR, k4, PTR, k4, *ws)
+    else:
+        raise ValueError(entry)
+    assert rc == 0, _native.last_error(lib)
+    return take(lib)
+
+
+# (B, Hq, Hk, M, N, D): many query heads per KV head over few rows, with
+# unaligned and whole score rows.
+@pytest.mark.parametrize("shape", [(64, 32, 1, 2, 4100, 64), (32, 16, 1, 3, 8192, 128),
+                                   (24, 64, 1, 8, 12001, 32), (40, 40, 2, 5, 5001, 16)])
+def test_scores_pack_at_most_eight_heads(lib, shape):
+    """The resident-Q scores kernel packs up to eight query heads of a KV head
+    (a power of two); more of them run as several groups and are not refused."""
+    a = make_args(*shape)
+    B, H, Hk, M, N, D = shape
+    rc = lib.fas_attention_scores(ctypes.byref(a), PTR, _native._I64x4(H * M * N, M * N, N, 1), None)
+    assert rc == 0, _native.last_error(lib)
+    sc = [f for name, f in take(lib) + launches(lib, "scores", a) if name == "scores"]
+    assert sc and all(f["pshift"] <= 3 and (H // Hk) % (1 << f["pshift"]) == 0 for f in sc)
