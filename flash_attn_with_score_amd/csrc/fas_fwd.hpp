@@ -520,7 +520,12 @@ void fwd_kernel(const FwdParams p) {
   // Staged score tile: row r (32 rows), 16-byte chunk ch (8 per row) at
   // unit r*8 + (ch ^ ((r >> 1) & 7)): conflict-free both for the MFMA-layout
   // writes (16 rows, one chunk) and the row-major reads (2 rows, 8 chunks).
-  auto stage_tile = [&](int base, const f32x16 (&sv)[2], bool masked)
+  // A stored score: 0 where the causal mask hides the key, and only there (a
+  // visible score of -inf stays -inf).
+  auto score_of = [&](float x, int key) __attribute__((always_inline)) {
+    return p.causal && key > p.causal_off + qpos ? 0.f : x * p.sm_scale;
+  };
+  auto stage_tile = [&](int base, const f32x16 (&sv)[2], int k0, bool masked)
                         __attribute__((always_inline)) {
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
@@ -529,7 +534,7 @@ void fwd_kernel(const FwdParams p) {
       float v[8];
       if (masked) {
 #pragma unroll
-        for (int e = 0; e < 8; ++e) v[e] = x[r0 + e] == neg_inf() ? 0.f : x[r0 + e] * p.sm_scale;
+        for (int e = 0; e < 8; ++e) v[e] = score_of(x[r0 + e], k0 + 16 * j + 8 * g + e);
       } else {
 #pragma unroll
         for (int e = 0; e < 8; ++e) v[e] = x[r0 + e] * p.sm_scale;
@@ -572,8 +577,7 @@ void fwd_kernel(const FwdParams p) {
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
           const int key = k0 + 32 * kb + acc_row(r, g);
-          const float x = s[kb][r];
-          if (key >= (p.N & ~7) && key < p.N) sr[key] = E::cvt(x == neg_inf() ? 0.f : x * p.sm_scale);
+          if (key >= (p.N & ~7) && key < p.N) sr[key] = E::cvt(score_of(s[kb][r], key));
         }
     }
   };
@@ -880,7 +884,7 @@ void fwd_kernel(const FwdParams p) {
         lds_barrier();
         if (act) {
           if (masked) apply_mask(s, k0);
-          stage_tile((loader ? wave : kOwnStg + pwave) * TSZ, s, masked);
+          stage_tile((loader ? wave : kOwnStg + pwave) * TSZ, s, k0, masked);
           if (masked) row_end(s, k0);
           update_offset_of(s);
           u32x4 pb[4];
@@ -927,7 +931,7 @@ void fwd_kernel(const FwdParams p) {
 
         if constexpr (MODE == kFwdScores) {
           if (loader) {
-            stage_tile((stage * NH + wave) * TSZ, s, masked);
+            stage_tile((stage * NH + wave) * TSZ, s, k0, masked);
           } else {
             // The storer reads this tile back row-major in the next key
             // tile (staged_pair), from other lanes of the same wave.  A
@@ -937,7 +941,7 @@ void fwd_kernel(const FwdParams p) {
             // closing lds_barrier (an asm with a memory clobber) keeps the
             // writes before the next iteration's read-back.
             __builtin_amdgcn_wave_barrier();
-            stage_tile((NW + pwave) * TSZ, s, masked);
+            stage_tile((NW + pwave) * TSZ, s, k0, masked);
           }
           if (masked) row_end(s, k0);
         }
@@ -966,8 +970,7 @@ void fwd_kernel(const FwdParams p) {
                 float y[8];
 #pragma unroll
                 for (int e = 0; e < 8; ++e) {
-                  const float x = s[j >> 1][8 * (j & 1) + e];
-                  y[e] = x == neg_inf() ? 0.f : x * p.sm_scale;
+                  y[e] = score_of(s[j >> 1][8 * (j & 1) + e], key + e);
                 }
                 const u32x4 w = {E::pack(y[0], y[1]), E::pack(y[2], y[3]), E::pack(y[4], y[5]),
                                  E::pack(y[6], y[7])};

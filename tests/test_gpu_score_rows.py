@@ -79,3 +79,40 @@ def test_unaligned_score_rows(case, dropout, gpu):
     assert torch.isfinite(got.float()).all()
     if not dropout:
         assert_out_close(o[:, heads], ref["out"][:, heads])
+
+
+# (Hq, Hk, M, N, D, causal): scores from the forward (few rows), the key-split
+# route, and the fused writer with 64-, 128- and 256-row blocks; unaligned rows.
+INF_CASES = [(4, 4, 3, 2048, 64, True), (8, 2, 8, 2050, 128, True), (4, 4, 2, 4096, 128, False),
+             (2, 2, 40, 4096, 64, True), (2, 2, 100, 200, 128, True), (2, 2, 70, 133, 64, True),
+             (130, 130, 100, 128, 16, True), (300, 300, 33, 96, 32, True)]
+
+
+@pytest.mark.parametrize("case", INF_CASES, ids=lambda c: "H{}K{}M{}N{}D{}{}".format(*c))
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16], ids=["f16", "bf16"])
+def test_visible_infinite_scores_stay(case, dtype, gpu):
+    """Keys of -inf and +inf scores (an infinite key element against q > 0):
+    0 where the causal mask hides them, and as they are wherever it does not,
+    in the diagonal's tile and in the last, partial tile too."""
+    import flash_attn_with_score_amd as fas
+
+    H, Hk, M, N, D, causal = case
+    print(f"[case] infinite scores {case} {dtype}", flush=True)
+    q, k, v = inputs.make_qkv(1, H, Hk, M, N, D, dtype=dtype, seed=8)
+    q[..., 0] = q[..., 0].abs() + 0.5
+    off = N - M
+    for key, sign in ((5, -1), (64, 1), (off // 2, -1), (off, -1), (off + M // 2, -1), (N - 1, -1)):
+        k[:, :, key, 0] = sign * float("inf")
+    _, s = fas.attention_with_scores(q.to(gpu), k.to(gpu), v.to(gpu), causal=causal)
+    torch.cuda.synchronize()
+    # Infinite products and finite ones add up to the same infinity in any order.
+    heads = sorted({0, 1, H - 1})
+    want = torch.matmul(q[:, heads].float(),
+                        k[:, [h // (H // Hk) for h in heads]].float().transpose(-1, -2)) * D ** -0.5
+    if causal:
+        i, j = torch.arange(M)[:, None] + off, torch.arange(N)[None]
+        want = want.masked_fill(j > i, 0.0)
+    got = s[:, heads].float().cpu()
+    inf = torch.isinf(want)
+    assert inf.any() and torch.equal(got[inf], want[inf])
+    assert_scores_close(s[:, heads].cpu().masked_fill(inf, 0.0), want.masked_fill(inf, 0.0))
