@@ -1084,10 +1084,12 @@ static int check_scores_out(const char* fn, const void* scores, const int64_t* s
 
 // Whether every score row starts on a 64-byte boundary (and ends on a 16-byte
 // one): the kernels then stream whole half-lines past the caches, otherwise
-// through them (store_score16 has both sides measured).
+// through them (store_score16 has both sides measured).  Those instances size
+// a block of rows by its pitch, so rows closer than n (M = 1 with any row
+// stride) take the others, which end each row at n.
 static int score_rows_aligned(const void* scores, const int64_t* st, int64_t n) {
   return (reinterpret_cast<uintptr_t>(scores) & 63u) == 0 && st[0] % 32 == 0 && st[1] % 32 == 0 &&
-         st[2] % 32 == 0 && n % 8 == 0;
+         st[2] % 32 == 0 && st[2] >= n && n % 8 == 0;
 }
 
 // Scores alone through the scores-only kernel; mask selects the causal /

@@ -116,3 +116,36 @@ def test_visible_infinite_scores_stay(case, dtype, gpu):
     inf = torch.isinf(want)
     assert inf.any() and torch.equal(got[inf], want[inf])
     assert_scores_close(s[:, heads].cpu().masked_fill(inf, 0.0), want.masked_fill(inf, 0.0))
+
+
+# (B, Hq, Hk, N, D): the fused writer, the forward's own scores, the resident-Q
+# kernel behind a key split, and (scores alone) the K-resident kernel.
+ONE_ROW = [(1, 4, 4, 256, 64), (2, 2, 1, 2048, 32), (64, 64, 1, 4096, 16)]
+
+
+@pytest.mark.parametrize("case", ONE_ROW, ids=lambda c: "B{}H{}K{}N{}D{}".format(*c))
+@pytest.mark.parametrize("row_stride", [0, 32])
+@pytest.mark.parametrize("alone", [False, True], ids=["attention", "alone"])
+def test_one_row_any_row_stride(case, row_stride, alone, gpu):
+    """M = 1: the row stride has no meaning, also below N."""
+    B, Hq, Hk, N, D = case
+    print(f"[case] one row {case} stride {row_stride} alone={alone}", flush=True)
+    lib = _native.load()
+    q, k, v = inputs.make_qkv(B, Hq, Hk, 1, N, D, dtype=torch.float16, seed=5)
+    qd, kd, vd = q.to(gpu), k.to(gpu), v.to(gpu)
+    args = _native.make_args(qd, kd, vd, torch.empty_like(qd), True, D ** -0.5)
+    nbytes = lib.fas_workspace_bytes(_native.VARIANT_SCORES, ctypes.byref(args), 0)
+    ws = torch.empty(nbytes + 256, dtype=torch.uint8, device=gpu)
+    buf = torch.full((B, Hq, 1, N), float("nan"), dtype=torch.float16, device=gpu)
+    st = _native._I64x4(Hq * N, N, row_stride, 1)
+    stream = torch.cuda.current_stream().cuda_stream
+    if alone:
+        rc = lib.fas_attention_scores(ctypes.byref(args), buf.data_ptr(), st, stream)
+    else:
+        rc = lib.fas_attention_with_scores(ctypes.byref(args), buf.data_ptr(), st,
+                                           ws.data_ptr() + (-ws.data_ptr()) % 256, nbytes, stream)
+    _native.check(lib, rc, "scores")
+    torch.cuda.synchronize()
+    heads = sorted({0, 1, Hq - 1})
+    ref = naive.reference_forward(q, k, v, causal=True, want=("scores",), heads=heads)
+    assert_scores_close(buf[:, heads], ref["scores"][:, heads])
