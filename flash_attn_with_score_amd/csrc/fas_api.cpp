@@ -421,17 +421,21 @@ struct Workspace {
 // (2 for at most 32 query rows per KV head, whose partials are small), up to
 // ~512 workgroups in all.  Depends on sizes only, so the workspace query and
 // the launch agree; fwd_plan picks the number of splits within it.
-// The scores variant writes its scores in a second kernel on this
-// route, so it splits only where the fused writer keeps few CUs busy for
-// long: from 2048 keys on (us, split against fused, B1 D128 causal: H4 M64
-// N1024 24 / 22; H4 M256 N1024 36 / 23; H12 M1024 N1024 44 / 24), up to 32
-// row blocks over 4096 keys when the key range is at least twice the query
-// range (H4 M2048 N4096 57 / 67; H1 M1024 N2048 41 / 37), up to 128 at 8
-// times (B2 H32 M512 N16384 607 / 734; H12
-// M1024 N4096 96 / 68), and up to 256 at 64 times (B8 H32 M256 N16384 1270 /
-// 1580).
+// The scores variant writes its scores in a second kernel on this route, so
+// it splits only where the fused writer keeps few CUs busy for long: from 2048
+// keys on (us, split against fused, B1 D128 causal: H4 M64 N1024 24 / 22; H4
+// M256 N1024 36 / 23; H12 M1024 N1024 44 / 24), up to 32 row blocks over 4096
+// keys when the key range is at least twice the query range (H4 M2048 N4096
+// 57 / 67; H1 M1024 N2048 41 / 37), up to 128 at 8 times (B2 H32 M512 N16384
+// 607 / 734; H12 M1024 N4096 96 / 68), and up to 256 at 64 times (B8 H32 M256
+// N16384 1270 / 1580).
+// With dropout the fused writer has 256-row blocks only and its step is the
+// random stream's products, which a split spreads over the CUs: up to 64 row
+// blocks whatever the keys (split / fused with dropout 0.1: B1 H1 S4096 D64 57
+// / 290, H4 M64 N1024 D64 33 / 48, H16 M1024 N4096 D128 157 / 316).
 static int64_t scores_split_max_wgs(const Problem& pr) {
   const int64_t m = pr.M, n = pr.N;
+  if (pr.dropout) return n >= 64 * m ? 256 : n >= 8 * m ? 128 : 64;
   if (n < 2048) return 0;
   return n >= 64 * m ? 256 : n >= 8 * m ? 128 : n >= 2 * m && n >= 4096 ? 32 : 0;
 }

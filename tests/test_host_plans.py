@@ -104,3 +104,17 @@ def test_scores_pack_at_most_eight_heads(lib, shape):
     assert rc == 0, _native.last_error(lib)
     sc = [f for name, f in take(lib) + launches(lib, "scores", a) if name == "scores"]
     assert sc and all(f["pshift"] <= 3 and (H // Hk) % (1 << f["pshift"]) == 0 for f in sc)
+
+
+# (B, Hq, Hk, M, N, D) with at most 64 row blocks of 256
+@pytest.mark.parametrize("shape", [(1, 1, 1, 4096, 4096, 64), (1, 4, 4, 64, 1024, 64),
+                                   (1, 16, 16, 1024, 4096, 128), (1, 8, 2, 2048, 2048, 32),
+                                   (2, 12, 12, 48, 1600, 128)])
+def test_scores_with_dropout_split_keys(lib, shape):
+    """Few row blocks with dropout: a key-split forward and the scores-only
+    kernel, not the fused writer's 256-row blocks (split / fused, us: 57 / 290
+    at B1 H1 S4096 D64)."""
+    plan = launches(lib, "scores", make_args(*shape, dropout=0.1))
+    assert [(n, f.get("mode", PLAIN)) for n, f in plan] == [("fwd", PLAIN), ("scores", PLAIN)]
+    many = launches(lib, "scores", make_args(4, 32, 32, 1024, 1024, 64, dropout=0.1))
+    assert [f["mode"] for _, f in many] == [SCORES]
