@@ -414,31 +414,6 @@ struct Workspace {
   SplitPlan sp;  // the forward's key split (nsplit 1: none)
 };
 
-// Key split of the plain / row-sum forward.  When the row blocks of the
-// whole problem give fewer workgroups than the chip has CUs (short query
-// ranges against long key ranges: decode, last-window scoring), each row
-// block's key tiles may be dealt to several workgroups of at least 8 tiles
-// (2 for at most 32 query rows per KV head, whose partials are small), up to
-// ~512 workgroups in all.  Depends on sizes only, so the workspace query and
-// the launch agree; fwd_plan picks the number of splits within it.
-// The scores variant writes its scores in a second kernel on this route, so
-// it splits only where the fused writer keeps few CUs busy for long: from 2048
-// keys on (us, split against fused, B1 D128 causal: H4 M64 N1024 24 / 22; H4
-// M256 N1024 36 / 23; H12 M1024 N1024 44 / 24), up to 32 row blocks over 4096
-// keys when the key range is at least twice the query range (H4 M2048 N4096
-// 57 / 67; H1 M1024 N2048 41 / 37), up to 128 at 8 times (B2 H32 M512 N16384
-// 607 / 734; H12 M1024 N4096 96 / 68), and up to 256 at 64 times (B8 H32 M256
-// N16384 1270 / 1580).
-// With dropout the fused writer has 256-row blocks only and its step is the
-// random stream's products, which a split spreads over the CUs: up to 64 row
-// blocks whatever the keys (split / fused with dropout 0.1: B1 H1 S4096 D64 57
-// / 290, H4 M64 N1024 D64 33 / 48, H16 M1024 N4096 D128 157 / 316).
-static int64_t scores_split_max_wgs(const Problem& pr) {
-  const int64_t m = pr.M, n = pr.N;
-  if (pr.dropout) return n >= 64 * m ? 256 : n >= 8 * m ? 128 : 64;
-  if (n < 2048) return 0;
-  return n >= 64 * m ? 256 : n >= 8 * m ? 128 : n >= 2 * m && n >= 4096 ? 32 : 0;
-}
 // Most query rows of a KV head's group for the finer key splits.
 constexpr int64_t kFewRows = fas::kFwdFewMax;
 // Whether a problem has at most that many and runs the forward that keeps
@@ -447,6 +422,41 @@ constexpr int64_t kFewRows = fas::kFwdFewMax;
 bool few_rows(const Problem& pr) {
   return (int64_t)pr.G * pr.M <= fas::kFwdFewMax && pr.pack == pr.G && !pr.dropout && pr.N > 0 &&
          pr.M > 0;
+}
+
+// Key split of the plain / row-sum forward.  When the row blocks of the
+// whole problem give fewer workgroups than the chip has CUs (short query
+// ranges against long key ranges: decode, last-window scoring), each row
+// block's key tiles may be dealt to several workgroups of at least 8 tiles
+// (2 for at most 32 query rows per KV head, whose partials are small), up to
+// ~512 workgroups in all.  Depends on sizes only, so the workspace query and
+// the launch agree; fwd_plan picks the number of splits within it.
+// The scores variant writes its scores in a second kernel on this route, so
+// it splits only where the fused writer keeps few CUs busy for long.  Most row
+// blocks of 256 (us, split / fused with its best row block, causal; the ratio
+// hardly depends on D):
+//  * at least 8 keys a query row, from 2048 keys on: 128 (B2 H32 M512 N16384
+//    D128 607 / 734), at least 64 keys: 256 (B8 H32 M256 N16384 1270 / 1580);
+//  * other shapes: 24 from 3000 keys on (H1 M512 N3000 D128 44 / 54, H12 35 /
+//    39 with D64; H4 M2048 N2048 46 / 38), 32 from 4096 (H1 S4096 47 / 64, H12
+//    M700 56 / 68; H12 M1024 71 / 63), 64 from 16384 (H4 M4096 234 / 264);
+//  * up to 128 rows over 1536 to 2047 keys, D >= 64: 32 (H1 M48 N1536 D128 24 /
+//    29, H12 M100 N1600 27 / 31; D32 21 / 20, N1024 24 / 22);
+//  * few rows of so many heads that even the 64-row blocks need a second round
+//    (a KV head's heads share a workgroup here, not there): every row block,
+//    from 16 key tiles on (B64 H32/1 M1 N1000 D64 134 / 171).
+// With dropout the fused writer has 256-row blocks only and its step is the
+// random stream's products, which a split spreads over the CUs: up to 64 row
+// blocks whatever the keys (split / fused with dropout 0.1: B1 H1 S4096 D64 57
+// / 290, H4 M64 N1024 D64 33 / 48, H16 M1024 N4096 D128 157 / 316).
+static int64_t scores_split_max_wgs(const Problem& pr) {
+  const int64_t m = pr.M, n = pr.N;
+  if (pr.dropout) return n >= 64 * m ? 256 : n >= 8 * m ? 128 : 64;
+  if (few_rows(pr) && n > 960 && (int64_t)pr.B * pr.H * ((m + 63) / 64) > kCus) return 256;
+  if (n < 2048)
+    return n >= 1536 && n >= 8 * m && pr.D >= 64 && (int64_t)pr.G * m <= 128 ? 32 : 0;
+  if (n >= 8 * m) return n >= 64 * m ? 256 : 128;
+  return n >= 16384 ? 64 : n >= 4096 ? 32 : n >= 3000 ? 24 : 0;
 }
 // Bytes of the fp32 partials of a plan (O, offset, weight sum, row sum).
 size_t split_bytes(const Problem& pr, const SplitPlan& sp) {
@@ -1204,14 +1214,20 @@ static int attention_with_scores_impl(const fas_attn_args* a, void* scores, cons
   //    2048 keys or more, where two rounds of longest-first pairs balance
   //    (B1 H8 S4096 131.9 / 93.1 / 82.6; B1 H12 M2048 N4096, not square:
   //    132.5 / 80.2 / 101.5; unaligned rows, whose stores cost more, B1 H8
-  //    S4095: 173 / 142 / 170);
+  //    S4095: 173 / 142 / 170); up to D = 32, whose steps are cheaper than the
+  //    wait for the last row block, also for others while the second round
+  //    stays short (B2 H12 M700 N2048 D32 51 / 32 / 28; B1 H28 M1024 N4096 99 /
+  //    71.6 / 72.5);
   //  * 128 rows while those run in one round (B1 H32 S1024 full 41.2 / 31.4 /
   //    43.0; B1 H12 S2000 D64 full 61.8 / 39.1 / 59.5);
   //  * 128 rows in two rounds under a causal mask, whose mirror order balances
   //    them, for rows of 1024 keys or more (B1 H16 S4096 164 / 131 / 182; B1
   //    H32 S1280 50.2 / 37.5 / 51.8; B4 H32 S512 29.3 / 33.2 / 50.7), but when
   //    they fill both rounds only for longer ones (B1 H32 S2048 90.4 / 96.7 /
-  //    111; B1 H16 S3072 103.8 / 78.4);
+  //    111; B1 H16 S3072 103.8 / 78.4), and where the mask cuts little of the
+  //    rows (N - M above M / 2) only while the second round is short (D128 M1024
+  //    N2048: H36 73 / 65, H56 79 / 87; B4 H8 M2048 N4096 171 / 221, D32 153 /
+  //    181);
   //  * else 256 rows (B1 H32 S2048 full 94.9 / 124.3 / 163.5; B2 H16 S1536 D64
   //    full 45.1 / 53.7 / 60.7).
   // Grouped heads, which 256-row blocks pack, go one by one there too (packed /
@@ -1223,11 +1239,14 @@ static int attention_with_scores_impl(const fas_attn_args* a, void* scores, cons
     const int64_t heads = (int64_t)pr.B * pr.H;
     const int64_t n256 = heads * ((pr.M + 255) / 256), n128 = heads * ((pr.M + 127) / 128),
                   n64 = heads * ((pr.M + 63) / 64);
-    const bool square = pr.causal && pr.N - pr.M < pr.M / 4;
-    if (n64 <= cus || (n128 <= cus && square && pr.N >= 2048 && aligned))
+    const int64_t cut = (int64_t)pr.N - pr.M;  // keys that every row sees
+    const bool square = cut < pr.M / 4, short64 = pr.D <= 32 && n64 <= cus * 11 / 8;
+    if (n64 <= cus ||
+        (n128 <= cus && pr.causal && (square || short64) && pr.N >= 2048 && aligned))
       bm = 64;
     else if (n128 <= cus ||
-             (n256 <= cus && pr.causal && pr.N >= 1024 && (n128 <= cus * 7 / 4 || pr.N >= 3072)))
+             (n256 <= cus && pr.causal && pr.N >= 1024 &&
+              (cut > pr.M / 2 ? n128 <= cus * 11 / 8 : n128 <= cus * 7 / 4 || pr.N >= 3072)))
       bm = 128;
     if (bm != fas::kFwdRows) pw.pack = 1;
   }

@@ -118,3 +118,35 @@ def test_scores_with_dropout_split_keys(lib, shape):
     assert [(n, f.get("mode", PLAIN)) for n, f in plan] == [("fwd", PLAIN), ("scores", PLAIN)]
     many = launches(lib, "scores", make_args(4, 32, 32, 1024, 1024, 64, dropout=0.1))
     assert [f["mode"] for _, f in many] == [SCORES]
+
+
+# (B, Hq, Hk, M, N, D), the forward's mode, rows per block
+SCORES_PLANS = [
+    ((1, 1, 1, 4096, 4096, 128), PLAIN, None),   # 16 row blocks over 4096 keys: split
+    ((1, 4, 4, 512, 3000, 128), PLAIN, None),    # 8 over 3000
+    ((1, 4, 4, 2048, 2048, 128), SCORES, 64),    # 32 over 2048: fused
+    ((1, 12, 12, 1024, 4096, 64), SCORES, 64),   # 48 over 4096
+    ((1, 4, 4, 4096, 16384, 128), PLAIN, None),  # 64 over 16384
+    ((2, 12, 12, 48, 1600, 128), PLAIN, None),   # few rows over 1536 keys and more
+    ((2, 12, 12, 48, 1600, 32), SCORES, 64),
+    ((2, 12, 12, 48, 1024, 128), SCORES, 64),
+    ((64, 32, 1, 1, 1000, 64), FEW, None),       # 2048 heads: the fused writer needs 8 rounds
+    ((64, 32, 1, 1, 960, 64), SCORES, 256),
+    ((2, 12, 12, 700, 2048, 32), SCORES, 64),    # D = 32: 264 blocks of 64
+    ((2, 12, 12, 700, 2048, 128), SCORES, 128),
+    ((1, 28, 28, 1024, 4096, 32), SCORES, 128),  # 448 blocks of 64
+    ((4, 8, 8, 2048, 4096, 128), SCORES, 256),   # two full rounds of 128, the mask cuts little
+    ((1, 36, 36, 1024, 2048, 128), SCORES, 128),
+    ((1, 32, 32, 2048, 3072, 128), SCORES, 128),
+    ((1, 16, 16, 4096, 4096, 128), SCORES, 128),
+]
+
+
+@pytest.mark.parametrize("shape,mode,bm", SCORES_PLANS)
+def test_scores_route_and_row_blocks(lib, shape, mode, bm):
+    """Key split or fused writer, and the writer's row blocks, on both sides of
+    each measured line."""
+    name, f = launches(lib, "scores", make_args(*shape))[0]
+    assert name == "fwd" and f["mode"] == mode
+    if mode == SCORES:
+        assert f["bm"] == bm
