@@ -964,13 +964,17 @@ void fwd_kernel(const FwdParams p) {
               }
             } else {
               uint16_t* sr = p.scores + b * p.ss0 + qh * p.ss1 + (int64_t)qpos * p.ss2;
+              // The row's last visible key (one path, as score_of has; tiles
+              // without a mask compare nothing).
+              const int last = masked && p.causal ? p.causal_off + qpos : 0x7fffffff;
 #pragma unroll
               for (int j = 0; j < 4; ++j) {
                 const int key = k0 + 16 * j + 8 * g;
                 float y[8];
 #pragma unroll
                 for (int e = 0; e < 8; ++e) {
-                  y[e] = score_of(s[j >> 1][8 * (j & 1) + e], key + e);
+                  const float x = s[j >> 1][8 * (j & 1) + e];
+                  y[e] = key + e > last ? 0.f : x * p.sm_scale;
                 }
                 const u32x4 w = {E::pack(y[0], y[1]), E::pack(y[2], y[3]), E::pack(y[4], y[5]),
                                  E::pack(y[6], y[7])};
