@@ -590,11 +590,10 @@ int64_t bwd_nkb(const Problem& pr) { return ((int64_t)pr.N + fas::kBwdBlock - 1)
 // written and read once (5 TB/s), about 6 us for the reduction, and about 3
 // tiles for each further workgroup's K and V loads and stores.  Estimated as
 // the forward's plan: the longest, or the mean over the CUs; at least 4 tiles
-// a piece for the longest block, at most 8 pieces, or G where the workspace
-// holds G partials.
-bool bwd_per_head(const Problem& pr) {
-  return pr.G > 1 && (int64_t)pr.B * pr.Hk * bwd_nkb(pr) < 256;
-}
+// a piece for the longest block, at most 8 pieces, or G where a workgroup per
+// key block and KV head leaves CUs idle: many query heads on few KV heads need
+// one piece per head (us of forward and backward, 8 pieces / G: B1 H64/1 S1024
+// D128 402 / 170, H32/1 S2048 D64 288 / 163).
 int bwd_pieces(const Problem& pr) {
   const int64_t nkb = bwd_nkb(pr), heads = (int64_t)pr.B * pr.Hk, n = heads * nkb;
   const int64_t rows = (pr.M + 63) / 64;
@@ -611,7 +610,7 @@ int bwd_pieces(const Problem& pr) {
   for (int64_t kb = 0; kb < nkb; ++kb) sum += (double)(heads * tiles(kb));
   int best = 1;
   double cost = 1e30;
-  const int most = bwd_per_head(pr) ? std::min(8, pr.G) : 8;
+  const int most = pr.G > 8 && n < 256 ? pr.G : 8;
   for (int s = 1; s <= most; ++s) {
     if (s > 1 && tiles(0) < 4 * s) break;
     const double longest = (double)((tiles(0) + s - 1) / s) + 3.0;
@@ -627,9 +626,6 @@ int bwd_pieces(const Problem& pr) {
   }
   return best;
 }
-// Partials the workspace holds: the launch's pieces, or one per query head
-// wherever G > 1 and B*Hk*nkb is below 256.
-int bwd_part_count(const Problem& pr) { return bwd_per_head(pr) ? pr.G : bwd_pieces(pr); }
 // The backward's stored dS (BwdParams.ds): 32-row block r sees 32-key blocks
 // [0, clamp(r + a, 0, ceil(N/32))): a = floor((N - M + 31) / 32) + 1 under the
 // causal mask (block (r, j) holds a visible pair iff (N - M) + 32 r + 31 >=
@@ -777,10 +773,11 @@ Workspace layout(int variant, const Problem& pr, int64_t split, size_t budget = 
     off += align256(rows);
     w.delta = off;
     off += align256(rows);
-    if (bwd_part_count(pr) > 1) {
+    const int pieces = bwd_pieces(pr);  // of the launch too: sizes alone decide
+    if (pieces > 1) {
       w.has_part = true;
       w.part = off;
-      off += align256((size_t)pr.B * pr.Hk * bwd_part_count(pr) * pr.N * 2 * pr.D * 4);
+      off += align256((size_t)pr.B * pr.Hk * pieces * pr.N * 2 * pr.D * 4);
     }
     // dS for the dQ kernel (2 bytes per visible pair, in 32 x 32 blocks),
     // when a head's blocks stay below 2 GiB, all of them within

@@ -168,10 +168,10 @@ def _ds_blocks(M, N, causal):
 
 
 def test_attention_backward_workspace(lib):
-    """Two (B*Hq, Mpad) fp32 row arrays, Mpad = M rounded up to 128, plus
-    per-query-head fp32 dK|dV partials only when Hq > Hk and the KV-head
-    grid B*Hk*ceil(N/128) is below 256 workgroups, plus 2 KiB per stored dS
-    block, which a query with split != 0 leaves out."""
+    """Two (B*Hq, Mpad) fp32 row arrays, Mpad = M rounded up to 128, plus one
+    fp32 dK|dV partial per KV head for each workgroup that a key block's row
+    tiles are dealt to, when there are several (grouped heads or not), plus
+    2 KiB per stored dS block, which a query with split != 0 leaves out."""
     def r256(x):
         return (x + 255) // 256 * 256
 
@@ -181,12 +181,15 @@ def test_attention_backward_workspace(lib):
     B, Hq, Hk, M, N, D = 2, 8, 2, 300, 500, 64
     a = make_args(B, Hq, Hk, M, N, D)
     mpad = 384
-    base = 2 * r256(B * Hq * mpad * 4) + r256(B * Hq * N * 2 * D * 4)
+    # 4 heads of 5 row tiles per key block and KV head: 5 pieces of 4 tiles.
+    base = 2 * r256(B * Hq * mpad * 4) + r256(B * Hk * 5 * N * 2 * D * 4)
     assert ws(a, 1) == base
     assert ws(a) == base + r256(B * Hq * _ds_blocks(M, N, True) * 2048)
-    a = make_args(64, 8, 4, 128, 128, 32)  # 64 * 4 * 1 = 256 workgroups: no partials
+    a = make_args(64, 8, 4, 128, 128, 32)  # two heads of two tiles: one piece
     assert ws(a, 1) == 2 * r256(64 * 8 * 128 * 4)
-    a = make_args(1, 4, 4, 100, 100, 128)  # MHA: no partials
+    a = make_args(1, 4, 4, 1024, 1024, 128)  # one head of 16 row tiles: 4 pieces of 4
+    assert ws(a, 1) == 2 * r256(4 * 1024 * 4) + r256(4 * 4 * 1024 * 2 * 128 * 4)
+    a = make_args(1, 4, 4, 100, 100, 128)  # two row tiles: one piece
     assert ws(a, 1) == 2 * r256(4 * 128 * 4)
     assert ws(a) == 2 * r256(4 * 128 * 4) + r256(4 * _ds_blocks(100, 100, True) * 2048)
 

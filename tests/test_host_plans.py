@@ -150,3 +150,29 @@ def test_scores_route_and_row_blocks(lib, shape, mode, bm):
     assert name == "fwd" and f["mode"] == mode
     if mode == SCORES:
         assert f["bm"] == bm
+
+
+# (B, Hq, Hk, S, D, causal), pieces
+PIECES = [
+    ((1, 64, 1, 1024, 128, 1), 52),  # up to one per query head
+    ((1, 32, 1, 2048, 64, 1), 32),
+    ((1, 16, 1, 2048, 128, 0), 16),
+    ((1, 8, 4, 2048, 64, 1), 8),     # more than the group's heads
+    ((1, 4, 4, 1024, 64, 1), 4),     # one head of 16 row tiles: at least 4 a piece
+    ((4, 32, 32, 4096, 64, 0), 1),   # the chip is full
+]
+
+
+@pytest.mark.parametrize("shape,pieces", PIECES)
+def test_dkdv_pieces(lib, shape, pieces):
+    """Workgroups per key block and KV head of the dK/dV kernel, and a
+    workspace that holds exactly their partials."""
+    B, Hq, Hk, S, D, causal = shape
+    a = make_args(B, Hq, Hk, S, S, D, causal)
+    (_, f), = launches(lib, "attention_backward", a)
+    assert f["pieces"] == pieces
+    r256 = lambda x: (x + 255) // 256 * 256  # noqa: E731
+    rows = 2 * r256(B * Hq * ((S + 127) // 128 * 128) * 4)
+    parts = r256(B * Hk * pieces * S * 2 * D * 4) if pieces > 1 else 0
+    assert lib.fas_workspace_bytes(_native.VARIANT_ATTENTION_BACKWARD, ctypes.byref(a), 1) == \
+        rows + parts
