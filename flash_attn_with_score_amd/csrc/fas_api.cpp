@@ -498,8 +498,10 @@ SplitPlan split_plan(const Problem& pr, bool top_left, int64_t max_wgs = 255,
 struct FwdPlan {
   int bm = fas::kFwdRows, nsplit = 1, tps = 0;
 };
-// The estimated end of each choice in steps of one 64-key tile per wave
-// (about 2 us at D = 128, 1 below), one workgroup at a time per CU:
+// The estimated end of each choice in steps of one 64-key tile per wave, one
+// workgroup at a time per CU, or two up to D = 32 without dropout (fwd_waves),
+// which then take 1.5 times as long a step (1.3 with the single wave of few
+// rows):
 //  * row blocks start longest first, so one round ends with the longest, two
 //    with the longest or with the last of the first round and the first of
 //    the second; never before the mean over the CUs;
@@ -507,22 +509,36 @@ struct FwdPlan {
 //    loads, epilogue), 3 with the merge of the 128-row blocks;
 //  * steps of the 128-row blocks move twice the K/V bytes per row, and a chip
 //    that runs evenly loaded clocks lower than one waiting for its longest
-//    row blocks: they count 1.35;
-//  * a key split adds the combine kernel: about 6 us, and its partials
-//    written and read back at 5 TB/s.
-// Measured (us, row-sum calls; 256 rows / 128 rows / split in two or eight):
-// B1 H32 S1024 D128 causal 34.3 / 24.1; S2048 59.9 / 49.2; S4096 147 / 168;
-// B1 H16 S4096 108 / 83; B1 H16 S2048 57.8 / 36.9 / 47.5; B2 H16 S1531 D64
-// full 33.7 / 40.1 / 49.4, causal 33.8 / 23.9; B1 H32/8 M200 N8000 195 / 111
-// / 45.4 (61.2 as 14 splits in two rounds); B1 H32 M256 N16384 388 / 236 /
-// 91.4 (105 as 16 splits in two rounds).
+//    row blocks: they count 1.2.  Up to 128 rows a 256-row block has one wave
+//    per SIMD and the pairs two: 1.5, and 1.8 with dropout, whose step (about
+//    3 us) is the VALU's;
+//  * a key split adds the combine kernel: about 6 us, 0.1 us a split (a row's
+//    splits are merged one after the other), and its partials written and
+//    read back at 5 TB/s.
+// Fitted to 1255 timed calls; the choice taken is 1.5% above the fastest in
+// the mean.  Measured (us, row-sum calls; 256 rows / 128 rows /
+// split): B1 H32 S1024 D128 causal 34.3 / 24.1; S2048 59.9 / 49.2; S4096 147 /
+// 168; B1 H16 S4096 108 / 83; B2 H16 S1531 D64 full 33.7 / 40.1 / 49.4, causal
+// 33.8 / 23.9; B4 H16 M1000 N6000 D16 89 / 74; B1 H32/8 M200 N8000 D128 195 /
+// 111 / 45.4 in eight (61.2 in 14, two rounds); B1 H8/1 M4 N32768 D16, in 32 /
+// 64 / 256: 21 / 22 / 47; B8 H32/8 M1 N32768 D16 in 4 / 8 (two a CU): 75 / 45;
+// dropout 0.1, B1 H32 M128 N1024 D64: 44 / 40 / 30 in two.
+// attention() (lse_out) also returns the log-normalizer, the same bits with and
+// without dropout for one query head per KV head (D <= 32: up to one workgroup
+// a CU): up to 128 rows all its calls take dropout's choice, above that none.
 FwdPlan fwd_plan(const Problem& pr, int pack, bool top_left, const SplitPlan& cap,
-                 bool key_pairs) {
+                 bool key_pairs, bool lse_out) {
   FwdPlan best;
   const int64_t cus = kCus, groups = (int64_t)pr.B * (pr.H / pack);
-  const int64_t n256 = groups * (((int64_t)pr.M * pack + 255) / 256);
+  const int64_t rows = (int64_t)pr.M * pack, n256 = groups * ((rows + 255) / 256);
   if (n256 == 0 || pr.N == 0 || n256 > 2 * cus) return best;
   const int64_t off = top_left ? 0 : (int64_t)pr.N - pr.M;
+  const bool few = (int64_t)pr.G * pr.M <= kFewRows;
+  const bool two = pr.D <= 32 && !pr.dropout;  // workgroups per CU
+  const double share = few ? 1.3 : 1.5;
+  const bool half = rows <= 128;
+  const bool drop_half = !few && (pr.dropout || lse_out) && pr.M <= 128;
+  const bool drop_full = !few && pr.dropout && !lse_out && pr.M > 128;
   // Steps of row block rb: its key tiles, or pairs of them.
   auto steps = [&](int64_t bm, int64_t rb) {
     int64_t hi = pr.N;
@@ -534,30 +550,37 @@ FwdPlan fwd_plan(const Problem& pr, int pack, bool top_left, const SplitPlan& ca
     return bm == 256 ? tiles : (tiles + 1) / 2;
   };
   auto makespan = [&](int64_t bm, double over) {
-    const int64_t nrb = ((int64_t)pr.M * pack + bm - 1) / bm, n = groups * nrb;
+    const int64_t nrb = (rows + bm - 1) / bm, n = groups * nrb;
     auto at = [&](int64_t i) { return (double)steps(bm, nrb - 1 - i / groups) + over; };
     double sum = 0;
     for (int64_t rb = 0; rb < nrb; ++rb) sum += (double)steps(bm, rb) + over;
-    double end = std::max(at(0), sum * (double)groups / (double)cus);
-    if (n > cus) end = std::max(end, at(cus - 1) + at(cus));
-    return end;
+    const double mean = sum * (double)groups / (double)cus;
+    if (two)  // the longest start beside the shortest
+      return std::max({at(0), 0.5 * share * mean, n > cus ? share * sum / (double)nrb : 0.0});
+    return std::max({at(0), mean, n > cus ? at(cus - 1) + at(cus) : 0.0});
   };
   double cost = makespan(256, 2.5);
   if (key_pairs && n256 <= cus) {
-    const double c = 1.35 * makespan(128, 3.0);
+    const double c =
+        (drop_half ? 1.8 : drop_full ? 1.1 : half || few ? 1.5 : 1.2) * makespan(128, 3.0);
     if (c < cost) {
       cost = c;
       best.bm = 128;
     }
   }
-  const int64_t nt = steps(256, ((int64_t)pr.M * pack + 255) / 256 - 1);
-  const double us_per_step = pr.D == 128 ? 2.0 : 1.0;
+  const int64_t nt = steps(256, (rows + 255) / 256 - 1);
+  const double us_per_step = drop_half ? 2.0 : drop_full ? 3.0 : few ? (pr.D == 128 ? 1.0 : 0.7)
+                             : pr.D == 128 ? 1.7 : 1.0;
   for (int64_t want = 2; want <= cap.nsplit; ++want) {
     const int64_t tps = (nt + want - 1) / want, ns = tps > 0 ? (nt + tps - 1) / tps : 0;
     if (ns != want) continue;
+    const int64_t n = n256 * ns;
+    const double rounds = !two       ? (double)((n + cus - 1) / cus)
+                          : n <= cus ? 1.0
+                                     : share * (double)((n + 2 * cus - 1) / (2 * cus));
     const double partials = (double)pr.B * pr.H * pr.M * (double)ns * (pr.D + 3) * 8;
-    const double c = (double)((n256 * ns + cus - 1) / cus) * ((double)tps + 2.5) +
-                     (6.0 + partials / 5e6) / us_per_step;
+    const double c =
+        rounds * ((double)tps + 2.5) + (6.0 + 0.1 * (double)ns + partials / 5e6) / us_per_step;
     if (c < cost) {
       cost = c;
       best.bm = 256;
@@ -850,8 +873,8 @@ T* at(void* ws, size_t off) {
 
 // Row blocks and key split of a plain or row-sum forward, with its partials.
 void apply_plan(fas::FwdParams& p, const Problem& pr, bool top_left, const Workspace& w, void* ws,
-                bool key_pairs = true) {
-  const FwdPlan f = fwd_plan(pr, p.pack, top_left, w.sp, key_pairs);
+                bool key_pairs = true, bool lse_out = false) {
+  const FwdPlan f = fwd_plan(pr, p.pack, top_left, w.sp, key_pairs, lse_out);
   p.bm = f.bm;
   p.nrb = (int)(((int64_t)pr.M * p.pack + f.bm - 1) / f.bm);
   if (f.nsplit == 1) return;
@@ -1373,7 +1396,7 @@ int fas_attention_forward(const fas_attn_args* a, float* lse, const int64_t st[3
   if ((rc = check_keep(fn, a, pr, &kl))) return rc;
   fas::FwdParams p = fwd_params(a, pr, false, fas::kFwdRows);
   rescale_dropout(p, a);
-  apply_plan(p, pr, false, w, ws);
+  apply_plan(p, pr, false, w, ws, true, true);
   p.lse_ln = lse;
   p.sl0 = st[0];
   p.sl1 = st[1];

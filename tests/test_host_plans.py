@@ -83,6 +83,8 @@ def launches(lib, entry, a, split=0):
     elif entry == "cross_softmax_sum":
         rc = lib.fas_attention_cross_token_softmax_sum(ref, split, PTR,
                                                        _native._I64x3(Hk * split, split, 1), *ws)
+    elif entry == "attention_forward":
+        rc = lib.fas_attention_forward(ref, PTR, rows, *ws)
     elif entry == "attention_backward":
         rc = lib.fas_attention_backward(ref, PTR, q4, PTR, rows, PTR, q4, PTR, k4, PTR, k4, *ws)
     else:
@@ -176,3 +178,40 @@ def test_dkdv_pieces(lib, shape, pieces):
     parts = r256(B * Hk * pieces * S * 2 * D * 4) if pieces > 1 else 0
     assert lib.fas_workspace_bytes(_native.VARIANT_ATTENTION_BACKWARD, ctypes.byref(a), 1) == \
         rows + parts
+
+
+# entry, (B, Hq, Hk, M, N, D, causal, dropout), rows per block, splits
+FWD_PLANS = [
+    ("row_sum", (1, 4, 4, 1, 8192, 128, 1, 0.0), 256, 32),
+    ("row_sum", (1, 8, 1, 4, 32768, 32, 1, 0.0), 256, 57),     # not 256: the merge is serial
+    ("row_sum", (8, 32, 8, 1, 32768, 16, 1, 0.0), 256, 8),     # D <= 32: 512 workgroups at once
+    ("row_sum", (8, 32, 8, 1, 32768, 64, 1, 0.0), 256, 4),
+    ("row_sum", (4, 16, 16, 1000, 6000, 16, 0, 0.0), 128, 1),  # 512 blocks, one round
+    ("row_sum", (4, 16, 16, 1000, 6000, 128, 0, 0.0), 256, 1),
+    ("row_sum", (1, 4, 4, 128, 1024, 128, 1, 0.0), 256, 2),    # one wave per SIMD
+    ("row_sum", (1, 4, 4, 512, 1024, 128, 1, 0.0), 128, 1),
+    ("row_sum", (1, 32, 32, 128, 1024, 64, 1, 0.1), 256, 2),   # dropout: two CUs, not two waves
+    ("row_sum", (1, 32, 32, 128, 1024, 64, 1, 0.0), 128, 1),
+    ("softmax_col_sum", (1, 12, 12, 40, 1000, 32, 1, 0.1), 256, 2),
+    ("scores", (1, 4, 4, 64, 1024, 64, 1, 0.1), 256, 2),
+]
+
+
+@pytest.mark.parametrize("entry,shape,bm,nsplit", FWD_PLANS)
+def test_forward_plan(lib, entry, shape, bm, nsplit):
+    """Rows per workgroup and key splits of the forward around its measured lines."""
+    B, Hq, Hk, M, N, D, causal, dropout = shape
+    _, f = launches(lib, entry, make_args(B, Hq, Hk, M, N, D, causal, dropout))[0]
+    assert (f["bm"], f["nsplit"]) == (bm, nsplit)
+
+
+@pytest.mark.parametrize("M,N", [(1, 5000), (40, 1000), (127, 1090), (128, 4096), (129, 1090),
+                                 (300, 600), (640, 640), (1000, 1000)])
+@pytest.mark.parametrize("D", [32, 128])
+def test_attention_plan_does_not_depend_on_dropout(lib, M, N, D):
+    """attention()'s log-normalizer has the same bits with and without dropout
+    (one query head per KV head): the keys are dealt alike."""
+    plans = [launches(lib, "attention_forward", make_args(1, 2, 2, M, N, D, 1, p))[0][1]
+             for p in (0.0, 0.3)]
+    assert [plans[0][x] for x in ("bm", "nsplit", "tps")] == \
+        [plans[1][x] for x in ("bm", "nsplit", "tps")]
