@@ -1248,6 +1248,9 @@ static int attention_with_scores_impl(const fas_attn_args* a, void* scores, cons
   //    rows (N - M above M / 2) only while the second round is short (D128 M1024
   //    N2048: H36 73 / 65, H56 79 / 87; B4 H8 M2048 N4096 171 / 221, D32 153 /
   //    181);
+  //  * 128 rows in two full rounds up to D = 32 for rows more than twice as
+  //    long as the query range (H32 M2048 N8192 D32 241 / 231, full 250 / 232,
+  //    H32/8 278 / 232; D128 338 / 360);
   //  * else 256 rows (B1 H32 S2048 full 94.9 / 124.3 / 163.5; B2 H16 S1536 D64
   //    full 45.1 / 53.7 / 60.7).
   // Grouped heads, which 256-row blocks pack, go one by one there too (packed /
@@ -1261,12 +1264,14 @@ static int attention_with_scores_impl(const fas_attn_args* a, void* scores, cons
                   n64 = heads * ((pr.M + 63) / 64);
     const int64_t cut = (int64_t)pr.N - pr.M;  // keys that every row sees
     const bool square = cut < pr.M / 4, short64 = pr.D <= 32 && n64 <= cus * 11 / 8;
+    const bool long32 = pr.D <= 32 && cut > pr.M && n128 >= cus * 7 / 4;
     if (n64 <= cus ||
         (n128 <= cus && pr.causal && (square || short64) && pr.N >= 2048 && aligned))
       bm = 64;
     else if (n128 <= cus ||
-             (n256 <= cus && pr.causal && pr.N >= 1024 &&
-              (cut > pr.M / 2 ? n128 <= cus * 11 / 8 : n128 <= cus * 7 / 4 || pr.N >= 3072)))
+             (n256 <= cus && pr.N >= 1024 &&
+              (pr.causal && cut <= pr.M / 2 ? n128 <= cus * 7 / 4 || pr.N >= 3072
+                                            : (pr.causal && n128 <= cus * 11 / 8) || long32)))
       bm = 128;
     if (bm != fas::kFwdRows) pw.pack = 1;
   }

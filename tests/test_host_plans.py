@@ -138,6 +138,8 @@ SCORES_PLANS = [
     ((2, 12, 12, 700, 2048, 128), SCORES, 128),
     ((1, 28, 28, 1024, 4096, 32), SCORES, 128),  # 448 blocks of 64
     ((4, 8, 8, 2048, 4096, 128), SCORES, 256),   # two full rounds of 128, the mask cuts little
+    ((1, 32, 8, 2048, 8192, 32), SCORES, 128),   # D = 32: longer rows than that
+    ((1, 32, 8, 2048, 8192, 64), SCORES, 256),
     ((1, 36, 36, 1024, 2048, 128), SCORES, 128),
     ((1, 32, 32, 2048, 3072, 128), SCORES, 128),
     ((1, 16, 16, 4096, 4096, 128), SCORES, 128),
