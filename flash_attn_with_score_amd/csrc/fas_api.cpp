@@ -328,68 +328,57 @@ struct SplitPlan {
   int64_t mpad = 0;
 };
 
-// Head split of the softmax column pass (ColsmParams.fold / nsplit): one
-// workgroup per (unit, split, output group), a unit being a mirror pair of
-// 256-key blocks (colsm64_kernel) or one key block (the buffered pass).
-// With fold heads per output column, nsplit workgroups share a unit's heads
-// (equal runs of their steps; the buffered pass: heads s, s + nsplit, ...) and
-// fold their column sums through partials and a ticket per unit; nsplit is the smallest of least cost, cost = rounds of
-// `slots` concurrent workgroups x heads per workgroup, so a problem with few
-// output groups still fills the chip (B1 with 4 KV heads of 7 query heads:
-// 7 splits, 224 workgroups), and one that fills it walks all of a KV head's
-// query heads per workgroup with its keys resident (8 KV heads of 4 query
-// heads at 16K keys: 256 workgroups, no split).
+// Split of the softmax column pass (ColsmParams.fold / nsplit): one workgroup
+// per (unit, split, output group), a unit being a mirror pair of 256-key blocks
+// (colsm64_kernel) or one key block (the buffered pass).  With fold heads per
+// output column, nsplit workgroups share a unit's heads and fold their column
+// sums through partials and a ticket per unit.
+// The buffered pass deals whole heads (s, s + nsplit, ...): nsplit is the
+// smallest of least cost, cost = rounds of `slots` concurrent workgroups x heads
+// per workgroup.
+// The recomputing pass deals equal runs of (head, 128-row step) pairs, any
+// number up to one a head, or one for 2 steps of the longest block: cost =
+// rounds x (steps of a workgroup + 5 for its K loads and the fold).  With a head's steps as the
+// unit, most shapes left CUs idle or took a round more (us of the call, D128
+// causal, multiples of the head split / any: B2 H28/4 S1531 92.8 / 82 in 10
+// instead of 21; B1 H32 S3000 split 2250 126 / 116 in 1 instead of 3; B1 H28/4
+// S4096 in 8 instead of 7, 256 workgroups).
 struct ColPlan {
   int fold = 1, nsplit = 1;
   int64_t nunits = 0, ngroups = 0;
 };
 constexpr int64_t kCus = 256;  // MI355X compute units
-// Where that leaves CUs idle, the recomputing pass also splits its row steps
-// (128 rows of one head), to pieces of at least 2 of them: cost = rounds x
-// (steps of a workgroup + 3 for its K loads and the fold).
-ColPlan col_plan(const Problem& pr, bool buffered, int64_t ncols, bool fold_heads,
-                 int64_t row_lo, bool split_rows) {
+// split_rows: false deals whole heads only (less room for partials).
+ColPlan col_plan(const Problem& pr, bool buffered, int64_t ncols, int64_t row_lo,
+                 bool split_rows) {
   ColPlan c;
-  c.fold = fold_heads ? pr.G : 1;
-  c.ngroups = (int64_t)pr.B * (pr.H / c.fold);
-  int64_t slots = kCus;  // colsm64_kernel: one 8-wave workgroup per CU
+  c.fold = pr.G;
+  c.ngroups = (int64_t)pr.B * pr.Hk;
+  const int64_t slots = buffered ? 8 * kCus : kCus;  // workgroups at once (4 or 8 waves)
+  const int64_t nkb = (ncols + 255) / 256;
   if (buffered) {
     const int64_t bk = ncols % 4 == 0 ? 256 : 64;  // keys per workgroup (VEC or not)
     c.nunits = (ncols + bk - 1) / bk;
-    slots = 8 * kCus;  // 4-wave workgroups, eight per CU
   } else {
-    c.nunits = ((ncols + 255) / 256 + 1) / 2;
+    c.nunits = (nkb + 1) / 2;
   }
-  int64_t best = INT64_MAX;
-  for (int ns = 1; ns <= c.fold; ++ns) {
-    const int64_t wgs = c.nunits * ns * c.ngroups;
-    const int64_t cost = ((wgs + slots - 1) / slots) * ((c.fold + ns - 1) / ns);
-    if (cost < best) {
-      best = cost;
-      c.nsplit = ns;
-    }
-  }
-  if (buffered || !fold_heads || !split_rows) return c;
-  // Steps of a unit's longest pair of blocks over the fold's heads.
+  const int64_t wgs = c.nunits * c.ngroups;
+  const bool heads = buffered || !split_rows;
+  // Steps of key block kb over the fold's heads (of a pair: first and last).
   auto steps = [&](int64_t kb) {
     int64_t lo = row_lo;
     if (pr.causal) lo = std::max<int64_t>(lo, 256 * kb - ((int64_t)pr.N - pr.M));
-    return std::max<int64_t>(0, (pr.M + 127) / 128 - std::max<int64_t>(0, lo) / 128);
+    return c.fold * std::max<int64_t>(0, (pr.M + 127) / 128 - std::max<int64_t>(0, lo) / 128);
   };
-  const int64_t nkb = (ncols + 255) / 256;
-  if (nkb == 0) return c;
-  const int64_t total = c.fold * (steps(0) + (nkb > 1 ? steps(nkb - 1) : 0));
-  const int64_t wgs = c.nunits * c.ngroups;
-  const int heads = c.nsplit;
-  auto cost_of = [&](int64_t ns) {
-    return ((wgs * ns + slots - 1) / slots) * ((total + ns - 1) / ns + 3);
-  };
-  best = cost_of(heads);
-  for (int m = 2; m <= 8; ++m) {
-    const int64_t ns = (int64_t)heads * m;
-    if (c.fold * steps(0) < 2 * ns) break;
-    if (cost_of(ns) < best) {
-      best = cost_of(ns);
+  const int64_t first = steps(0), total = first + (nkb > 1 ? steps(nkb - 1) : 0);
+  const int64_t work = heads ? c.fold : total, over = heads ? 0 : 5;
+  const int64_t most =
+      heads ? c.fold : std::max<int64_t>(c.fold, std::min<int64_t>(8 * c.fold, first / 2));
+  int64_t best = INT64_MAX;
+  for (int64_t ns = 1; ns <= most; ++ns) {
+    const int64_t cost = ((wgs * ns + slots - 1) / slots) * ((work + ns - 1) / ns + over);
+    if (cost < best) {
+      best = cost;
       c.nsplit = (int)ns;
     }
   }
@@ -753,10 +742,10 @@ Workspace layout(int variant, const Problem& pr, int64_t split, size_t budget = 
     }
     const bool buffered = variant == FAS_VARIANT_CROSS_SOFTMAX_SUM_BUFFERED;
     const int64_t row_lo = variant == FAS_VARIANT_SOFTMAX_COL_SUM ? 0 : split;
-    w.cp = col_plan(pr, buffered, ncols, true, row_lo, true);
+    w.cp = col_plan(pr, buffered, ncols, row_lo, true);
     // Without room for that many partials, the heads' split alone.
     if (off + (size_t)w.cp.ngroups * (w.cp.nsplit * ncols + w.cp.nunits) * 4 + 512 > budget)
-      w.cp = col_plan(pr, buffered, ncols, true, row_lo, false);
+      w.cp = col_plan(pr, buffered, ncols, row_lo, false);
     if (w.has_few) w.cp.nsplit = 1;
     if (w.cp.nsplit > 1) {
       // The splits' column sums and one ticket per (output group, unit).

@@ -161,17 +161,20 @@ def test_metric_shape_softmax_col_sum(gpu):
 
 
 # The softmax column passes fold a KV head's G query heads inside the kernel:
-# one workgroup per key-block pair walking all G heads (nsplit 1), or the
-# heads dealt to nsplit workgroups (heads s, s + nsplit, ...) whose column
+# one workgroup per key-block pair walking all G heads (nsplit 1), or equal
+# runs of their (head, 128-row step) pairs on nsplit workgroups whose column
 # sums the last to finish adds through a device-scope ticket.  Shapes chosen
-# so the plan (tests/test_host.py::_col_plan, the host rule restated) takes
-# each regime, including uneven head sets (G = 3 over 2 splits, G = 7 over 4).
+# so the plan (tests/test_host.py::_col_plan, held against the library by
+# tests/test_host_plans.py) takes each regime: whole heads, runs of several
+# heads, runs that start and end inside a head.
 HEAD_SPLIT_CASES = [
     # (B, Hq, Hk, S, D, expected nsplit)
-    (4, 96, 32, 256, 64, 2),
-    (2, 224, 32, 256, 32, 4),
+    (4, 96, 32, 256, 64, 2),    # 3 heads of 2 steps: 3 steps each
+    (2, 224, 32, 256, 32, 4),   # 7 heads of 2 steps: 3 or 4
     (8, 64, 32, 256, 64, 1),
-    (1, 8, 2, 1024, 128, 4),
+    (1, 8, 2, 1024, 128, 14),   # 4 heads of 8 steps
+    (2, 9, 3, 900, 64, 10),     # 3 heads of 8 steps, ragged
+    (1, 14, 2, 700, 32, 19),    # 7 heads of 6 steps
 ]
 
 

@@ -94,32 +94,42 @@ def make_args(B=1, Hq=4, Hk=2, M=300, N=300, D=128, causal=1, dtype=0, ptr=0x100
     return a
 
 
-def _col_plan(B, Hq, Hk, ncols, buffered, cus=256):
-    """Head split of the softmax column pass, restated: the fold's G query
-    heads are dealt to nsplit workgroups per unit (a mirror pair of 256-key
-    blocks, or one key block of the buffered pass); nsplit is the smallest of
-    least cost, cost = rounds of concurrent workgroups x heads per workgroup.
+def _col_plan(B, Hq, Hk, ncols, buffered, M=None, N=None, causal=1, row_lo=0, cus=256):
+    """Split of the softmax column pass, restated (tests/test_host_plans.py holds
+    it against the library): the rows of the fold's G query heads are dealt to
+    nsplit workgroups per unit (a mirror pair of 256-key blocks, or one key block
+    of the buffered pass), whole heads in the buffered pass, else equal runs of
+    (head, 128-row step) pairs, up to one a head or one for two steps of the longest
+    block; nsplit
+    is the smallest of least cost, cost = rounds of concurrent workgroups x (heads
+    per workgroup, or steps per workgroup + 5).  M, N: ncols unless given.
     Returns (nsplit, units, output groups)."""
-    G = Hq // Hk
-    groups = B * Hk
+    G, M, N = Hq // Hk, M or ncols, N or ncols
+    groups, nkb = B * Hk, -(-ncols // 256)
     if buffered:
-        bk = 256 if ncols % 4 == 0 else 64
-        units, slots = -(-ncols // bk), 8 * cus
+        units, slots = -(-ncols // (256 if ncols % 4 == 0 else 64)), 8 * cus
+        work, over, most = G, 0, G
     else:
-        units, slots = (-(-ncols // 256) + 1) // 2, cus
-    cost = {ns: -(-(units * ns * groups) // slots) * -(-G // ns) for ns in range(1, G + 1)}
-    best = min(cost.values())
-    return min(ns for ns, c in cost.items() if c == best), units, groups
+        units, slots = (nkb + 1) // 2, cus
+
+        def steps(kb):
+            lo = max(row_lo, 256 * kb - (N - M)) if causal else row_lo
+            return G * max(0, -(-M // 128) - max(0, lo) // 128)
+
+        work, over = steps(0) + (steps(nkb - 1) if nkb > 1 else 0), 5
+        most = max(G, min(8 * G, steps(0) // 2))
+    cost = {ns: -(-(units * ns * groups) // slots) * (-(-work // ns) + over)
+            for ns in range(1, most + 1)}
+    return min(cost, key=lambda ns: (cost[ns], ns)), units, groups
 
 
 def test_col_plan_examples():
-    """The plan on the BASELINE shapes: 7 splits for 4 KV heads of 7 query
-    heads (224 workgroups instead of 32), none at 8 KV heads x 32 pairs (256
-    workgroups), one head per workgroup for the cross-token pass at split
-    12288 (768 workgroups in 3 rounds beat 192 in one round of 4 heads)."""
-    assert _col_plan(1, 28, 4, 4096, False) == (7, 8, 4)
+    """4 KV heads of 7 query heads at S = 4096: 256 workgroups; 8 KV heads x 32
+    pairs fill the chip unsplit; the cross-token pass at split 12288 in whole
+    rounds; 32 heads of 8 pairs: one workgroup a CU."""
+    assert _col_plan(1, 28, 4, 4096, False) == (8, 8, 4)
     assert _col_plan(1, 32, 8, 16384, False) == (1, 32, 8)
-    assert _col_plan(1, 32, 8, 12288, False) == (4, 24, 8)
+    assert _col_plan(1, 32, 8, 12288, False, 16384, 16384, 1, 12288) == (4, 24, 8)
     assert _col_plan(1, 32, 32, 4096, False) == (1, 8, 32)
     assert _col_plan(1, 32, 8, 12288, True) == (4, 48, 8)
 
@@ -130,8 +140,8 @@ def test_workspace_sizes(lib):
     def r256(x):
         return (x + 255) // 256 * 256
 
-    def folds(ncols, buffered):
-        ns, units, groups = _col_plan(B, Hq, Hk, ncols, buffered)
+    def folds(ncols, buffered, row_lo=0):
+        ns, units, groups = _col_plan(B, Hq, Hk, ncols, buffered, M, N, 1, row_lo)
         return 0 if ns == 1 else r256(groups * ns * ncols * 4) + r256(groups * units * 4)
 
     a = make_args(B, Hq, Hk, M, N, D)
@@ -144,13 +154,13 @@ def test_workspace_sizes(lib):
     assert folds(N, False) > 0  # 4 query heads per KV head, 4 workgroups unsplit: split
     assert ws(_native.VARIANT_SOFTMAX_COL_SUM) == r256(B * Hq * M * 4) + folds(N, False)
     assert ws(_native.VARIANT_CROSS_QK_SUM) == r256(B * Hk * ((M - split + 63) // 64 + 1) * D * 4)
-    assert ws(_native.VARIANT_CROSS_SOFTMAX_SUM) == r256(B * Hq * M * 4) + folds(split, False)
+    assert ws(_native.VARIANT_CROSS_SOFTMAX_SUM) == r256(B * Hq * M * 4) + folds(split, False, split)
     # The buffered region: fp16 exponents, then one fp32 offset per row and
     # 64-key tile.
     assert ws(_native.VARIANT_CROSS_SOFTMAX_SUM_BUFFERED) == (
         r256(B * Hq * M * 4) + folds(split, True) + r256(B * Hq * (M - split) * split * 2)
         + r256(B * Hq * (M - split) * ((split + 63) // 64) * 4))
-    # MHA needs no per-query-head partials.
+    # One head of 3 row steps per output column: not split.
     a1 = make_args(B, 4, 4, M, N, D)
     assert lib.fas_workspace_bytes(_native.VARIANT_SOFTMAX_COL_SUM, ctypes.byref(a1), 0) == \
         r256(B * 4 * M * 4)
@@ -249,8 +259,8 @@ def test_key_split_workspace(lib):
     ws = lambda v, s=0: lib.fas_workspace_bytes(v, ctypes.byref(a), s)  # noqa: E731
     assert ws(_native.VARIANT_ROW_SUM) == split
     assert ws(_native.VARIANT_ATTENTION_FORWARD) == split
-    ns, units, groups = _col_plan(B, Hq, Hk, N, False)
-    assert ns == 2
+    ns, units, groups = _col_plan(B, Hq, Hk, N, False, M, N)
+    assert ns == 2  # two heads of one 32-row step
     assert ws(_native.VARIANT_SOFTMAX_COL_SUM) == (
         r256(B * Hq * M * 4) + r256(groups * ns * N * 4) + r256(groups * units * 4) + split)
     assert ws(_native.VARIANT_SCORES) == split  # key-split forward + scores-only kernel

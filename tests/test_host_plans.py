@@ -9,6 +9,7 @@ from __future__ import annotations
 
 import ctypes
 import os
+import random
 import subprocess
 
 import pytest
@@ -217,3 +218,28 @@ def test_attention_plan_does_not_depend_on_dropout(lib, M, N, D):
              for p in (0.0, 0.3)]
     assert [plans[0][x] for x in ("bm", "nsplit", "tps")] == \
         [plans[1][x] for x in ("bm", "nsplit", "tps")]
+
+
+@pytest.mark.parametrize("seed", range(4))
+def test_column_pass_split(lib, seed):
+    """The column pass's workgroups per unit against the rule restated in
+    test_host, over shapes that leave CUs idle, fill them and take rounds."""
+    from tests.test_host import _col_plan
+
+    rng = random.Random(seed)
+    shapes = [(1, 28, 4, 4096, 4096, 0), (2, 28, 4, 1531, 1531, 0), (1, 32, 32, 3000, 3000, 2250),
+              (1, 8, 2, 1024, 1024, 0), (1, 2, 2, 1300, 1300, 0), (1, 16, 1, 3000, 3000, 0)]
+    for _ in range(60):
+        Hk, G = rng.choice([1, 2, 4, 8, 12, 32]), rng.choice([1, 2, 3, 4, 7, 8])
+        M, N = rng.randint(40, 5000), rng.randint(40, 5000)
+        shapes.append((rng.choice([1, 2, 4]), Hk * G, Hk, M, N, rng.choice([0, 0, rng.randint(1, N)])))
+    for B, Hq, Hk, M, N, split in shapes:
+        causal = rng.choice([0, 1])
+        a = make_args(B, Hq, Hk, M, N, 64, causal)
+        plan = launches(lib, "cross_softmax_sum" if split else "softmax_col_sum", a, split)
+        if plan[-1][0] != "colsm":  # few rows: their scores are kept
+            assert not split and Hq // Hk * M <= 32
+            continue
+        want = _col_plan(B, Hq, Hk, split or N, False, M, N, causal, split)[0]
+        assert plan[-1][1]["nsplit"] == want, (B, Hq, Hk, M, N, causal, split)
+        assert plan[-1][1]["fold"] == Hq // Hk
