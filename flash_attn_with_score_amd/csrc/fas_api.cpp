@@ -714,8 +714,11 @@ int64_t ncols_of(int variant, const Problem& pr, int64_t split) {
   }
 }
 
-// budget: largest total the caller can provide (SIZE_MAX: any); only the
-// key-split partials adapt to it, by a smaller split.
+constexpr size_t kFewMaxBytes = (size_t)4 << 30;
+
+// budget: largest total the caller can provide (SIZE_MAX: any).  The kept
+// scores, the column pass's partials, the keep bits and the stored dS are left
+// out where they do not fit; the key-split partials take a smaller split.
 Workspace layout(int variant, const Problem& pr, int64_t split, size_t budget = SIZE_MAX) {
   Workspace w;
   size_t off = 0;
@@ -730,11 +733,18 @@ Workspace layout(int variant, const Problem& pr, int64_t split, size_t budget = 
     w.lse = off;
     off += align256((size_t)pr.B * pr.H * pr.M * 4);
     // Few query rows: their scores, fp32, kept by the forward for the column
-    // sums (rows padded to whole key tiles), when they fit the budget.
+    // sums (rows padded to whole key tiles; at most 128 bytes a key and KV
+    // head, where K and V are 4 D).  Only up to kFewMaxBytes, and where the
+    // budget leaves the key split half the splits the forward would take: one
+    // with fewer costs what the column pass over K does (B8 H32/8 M1 N32768
+    // D128, four splits: 250 us, in two 329, unsplit 556; the pass over K 590)
+    // and more where few row blocks need many splits.
     if (variant == FAS_VARIANT_SOFTMAX_COL_SUM && few_rows(pr)) {
       const size_t bytes =
           align256((size_t)pr.B * pr.H * pr.M * (((size_t)pr.N + 63) / 64 * 64) * 4);
-      if (off + bytes <= budget) {
+      const int want = fwd_plan(pr, pr.pack, false, split_plan(pr, false), false, false).nsplit;
+      if (bytes <= kFewMaxBytes && off + bytes <= budget &&
+          2 * split_plan(pr, false, 255, budget - off - bytes).nsplit >= want) {
         w.has_few = true;
         w.few = off;
         off += bytes;

@@ -195,8 +195,10 @@ int fas_attention_with_softmax_col_sum(const fas_attn_args* a, float* col_sum,
  * caller still passes the inputs and outputs; nothing is allocated or freed,
  * here or in any library routine this call makes.
  * Limits: the array holds 64 MiB per GPU (B*Hq*M*4 bytes of row normalizers,
- * + B*Hq*N*4 of group partials when Hq > Hk, + key-split partials, which
- * shrink to fit); larger problems return FAS_ERR_WORKSPACE.  Every call on
+ * + the column pass's partials, + key-split partials and few rows' kept
+ * scores, which shrink or are left out to fit); problems whose normalizers
+ * and whole-head column partials alone are larger return
+ * FAS_ERR_WORKSPACE.  Every call on
  * one GPU shares that GPU's array: calls that overlap on one GPU (other
  * streams, other host threads) race and must be serialised by the caller.
  * No part of the array needs to start at zero; each call writes what it

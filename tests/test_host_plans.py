@@ -34,7 +34,7 @@ def lib(tmp_path_factory):
                        check=True, capture_output=True, text=True)
     so = str(tmp / "plans.so")
     subprocess.run([fas_build.hipcc(), "-shared", "-fPIC", f"--offload-arch={fas_build.ARCH}",
-                    *objs, "-o", so], check=True, capture_output=True, text=True)
+                    "-Wl,-Bsymbolic", *objs, "-o", so], check=True, capture_output=True, text=True)
     lib = ctypes.CDLL(so)
     for name, (restype, argtypes) in _native._SIGNATURES.items():
         fn = getattr(lib, name)
@@ -70,7 +70,7 @@ def launches(lib, entry, a, split=0):
     q4, k4 = a.q_stride, a.k_stride
     rows, keys = _native._I64x3(H * M, M, 1), _native._I64x3(Hk * N, N, 1)
     s4 = _native._I64x4(H * M * N, M * N, N, 1)
-    variant = getattr(_native, "VARIANT_" + entry.upper())
+    variant = getattr(_native, "VARIANT_" + entry.upper().replace("_NOALLOC", ""))
     nbytes = lib.fas_workspace_bytes(variant, ctypes.byref(a), split)
     ws = (PTR, nbytes, None)
     ref = ctypes.byref(a)
@@ -81,6 +81,8 @@ def launches(lib, entry, a, split=0):
         rc = lib.fas_attention_with_row_sum(ref, PTR, rows, *ws)
     elif entry == "softmax_col_sum":
         rc = lib.fas_attention_with_softmax_col_sum(ref, PTR, keys, *ws)
+    elif entry == "softmax_col_sum_noalloc":
+        rc = lib.fas_attention_with_softmax_col_sum_noalloc(ref, PTR, keys, None)
     elif entry == "cross_softmax_sum":
         rc = lib.fas_attention_cross_token_softmax_sum(ref, split, PTR,
                                                        _native._I64x3(Hk * split, split, 1), *ws)
@@ -243,3 +245,30 @@ def test_column_pass_split(lib, seed):
         want = _col_plan(B, Hq, Hk, split or N, False, M, N, causal, split)[0]
         assert plan[-1][1]["nsplit"] == want, (B, Hq, Hk, M, N, causal, split)
         assert plan[-1][1]["fold"] == Hq // Hk
+
+
+# (B, Hq, Hk, M, N), whether the scores are kept, least splits
+NOALLOC = [((8, 32, 8, 1, 8192), 1, 4), ((8, 32, 8, 1, 32768), 1, 4), ((8, 32, 8, 1, 60000), 0, 4),
+           ((1, 32, 8, 1, 400000), 1, 16), ((1, 32, 8, 1, 500000), 0, 32),
+           ((1, 8, 8, 4, 500000), 1, 16)]
+
+
+@pytest.mark.parametrize("shape,kept,nsplit", NOALLOC)
+def test_kept_scores_leave_room_for_the_split(lib, shape, kept, nsplit):
+    """In 64 MiB of scratch, few rows' scores are kept only where the key split's
+    partials fit beside them: near the limit the forward keeps its splits."""
+    plan = launches(lib, "softmax_col_sum_noalloc", make_args(*shape, 128))
+    (name, f), second = plan
+    assert name == "fwd" and f["kept"] == kept and f["mode"] == (FEW if kept else PLAIN)
+    assert second[0] == ("few_cols" if kept else "colsm")
+    assert f["nsplit"] >= nsplit
+
+
+def test_kept_scores_stay_below_4_gib(lib):
+    """Kept scores of 4 GiB and less; past that the column pass reads K."""
+    below, past = ((64, 32, 8, 1, n, 128) for n in (524288, 524352))
+    for shape, kept in ((below, 1), (past, 0)):
+        a = make_args(*shape)
+        assert launches(lib, "softmax_col_sum", a)[0][1]["kept"] == kept
+    nbytes = lib.fas_workspace_bytes(_native.VARIANT_SOFTMAX_COL_SUM, ctypes.byref(a), 0)
+    assert nbytes < 1 << 30
