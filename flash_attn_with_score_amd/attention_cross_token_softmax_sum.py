@@ -13,12 +13,21 @@ from . import _common, _native
 
 __all__ = ["attention_cross_token_softmax_sum", "attention_cross_token_softmax_sum_buffered"]
 
-# The buffered variant keeps the region's scores only for at most
-# BUFFERED_ROWS query rows past the split over at most BUFFERED_KEYS keys, where
-# a column pass of its own costs more than the little it writes (us, buffered /
-# recomputed, D128: B4 H4 S296 split 250 23.4 / 24.6, split 232 20.6 / 24.5; B1
-# H12 S704 split 640 34.3 / 32.0; B1 H32 S2048 split 2000 79.5 / 63.0).
-BUFFERED_ROWS, BUFFERED_KEYS = 64, 512
+# The buffered variant keeps the region's scores only where that is faster than
+# a second pass over K: at most BUFFERED_ROWS query rows past the split over at
+# most BUFFERED_KEYS keys whose region rows start on 16 bytes, or twice the rows
+# at any split over at most BUFFERED_SHORT keys.  Time kept / recomputed, mean over six head
+# counts and D = 32, 64, 128 (fp16, causal), 64 rows: S 200 0.96, 296 0.95, 384
+# 0.90, 448 1.00, 512 1.04; 8 rows 0.83, 0.82, 0.83, 0.92, 0.97; 128 rows 1.02
+# to 1.09; splits that are no multiple of 8, 33 rows: S 136 0.91, 200 1.08, 296
+# 1.10, 384 1.14, 448 1.32, 512 1.45.
+BUFFERED_ROWS, BUFFERED_KEYS, BUFFERED_SHORT = 64, 448, 160
+
+
+def _keeps_region(M: int, N: int, split: int) -> bool:
+    if N <= BUFFERED_SHORT:
+        return M - split <= 2 * BUFFERED_ROWS
+    return M - split <= BUFFERED_ROWS and N <= BUFFERED_KEYS and split % 8 == 0
 
 
 def attention_cross_token_softmax_sum_buffered(
@@ -34,13 +43,11 @@ def attention_cross_token_softmax_sum_buffered(
 
     The reference's pass 1 stores the raw scores, B * Hq * M * N * 4 bytes
     (:704-705), and its pass 2 reloads them.  On MI355X recomputing q . k for
-    the region (queries >= split, keys < split) is faster than writing and reading even 2 bytes per score of it
-    (fas_attention_cross_token_softmax_sum_buffered: B1 H32/8 S16384 split
-    12288 D128 2.94 against 2.35 ms, B1 H32 S4096 split 3072 231 against 190
-    us, split 3001 560 against 193 us, B1 H4 S1664 split 283 D32 151 against
-    53 us), is exact to fp32 instead of fp16 exponents, and needs no region,
-    so this entry point recomputes too, but for the few rows of
-    BUFFERED_ROWS.
+    the region (queries >= split, keys < split) is faster than writing and
+    reading even 2 bytes per score of it, is exact to fp32 instead of fp16
+    exponents, and needs no region, so this entry point recomputes too, but for
+    the small regions of _keeps_region
+    (fas_attention_cross_token_softmax_sum_buffered).
     """
     Dq, Dk, Dv = q.shape[-1], k.shape[-1], v.shape[-1]
     assert Dq == Dk == Dv, "Q, K, V must have the same head_dim"
@@ -62,7 +69,7 @@ def attention_cross_token_softmax_sum_buffered(
     # The reference's buffered kernel ignores dropout_p and draws no seed.
     args = _native.pack_args(p.q, p.k, p.v, output, causal, p.sm_scale)
     variant, entry = _native.VARIANT_CROSS_SOFTMAX_SUM, "fas_attention_cross_token_softmax_sum"
-    if M - split <= BUFFERED_ROWS and N <= BUFFERED_KEYS:
+    if _keeps_region(M, N, split):
         variant, entry = _native.VARIANT_CROSS_SOFTMAX_SUM_BUFFERED, entry + "_buffered"
     ws_ptr, ws_bytes, ws = _common.workspace(variant, args, split, q.device)
     _common.call(entry, p.q, args, int(split), cross.data_ptr(), _native.pack_strides(cross), ws_ptr,

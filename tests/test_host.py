@@ -461,3 +461,16 @@ def test_make_args_packs_every_field():
     assert (a.dropout_seed, a.dropout_offset) == (2**63 + 5, 2**40 + 7)
     b = _native.make_args(o, k, v, o, False, 0.5)
     assert (b.dtype, b.causal, b.dropout_p, b.dropout_seed, b.dropout_offset) == (1, 0, 0.0, 0, 0)
+
+
+@pytest.mark.parametrize("M,N,split,kept", [
+    (448, 448, 384, True), (448, 448, 376, False), (456, 456, 400, False),
+    (400, 400, 341, False), (400, 400, 344, True), (160, 160, 33, True), (160, 160, 31, False),
+    (161, 161, 133, False),
+    (40, 168, 8, True), (8, 400, 40, True)])
+def test_buffered_sum_keeps_small_regions(M, N, split, kept):
+    """Which calls of the buffered cross-token sum keep their region's scores:
+    both sides of each line, no rows past the split among them."""
+    from flash_attn_with_score_amd.attention_cross_token_softmax_sum import _keeps_region
+
+    assert _keeps_region(M, N, split) is kept
