@@ -57,7 +57,9 @@ WORKLOADS = {
     "col_softmax": ("attention_with_softmax_col_sum", False, "mfma", 6),
     "cross_qk": ("attention_cross_token_qk_sum", True, "mfma", 4),
     "cross_softmax": ("attention_cross_token_softmax_sum", True, "mfma", None),
-    "cross_softmax_buffered": ("attention_cross_token_softmax_sum_buffered", True, "hbm", None),
+    # Keeps its region's scores only where that is small (keeps_region), else
+    # the same work as cross_softmax.
+    "cross_softmax_buffered": ("attention_cross_token_softmax_sum_buffered", True, "mfma", None),
     # attention()'s forward pass (flash.py:32-169) with inputs that need
     # gradients, as in training: O and L, plus the dropout keep bits the
     # backward reads when dropout is on.
@@ -90,6 +92,13 @@ def cross_pairs(M: int, N: int, split: int, causal: bool, offset: int) -> int:
     return total
 
 
+def keeps_region(M: int, N: int, split: int) -> bool:
+    """Whether the buffered cross-token sum keeps its region's scores."""
+    from flash_attn_with_score_amd.attention_cross_token_softmax_sum import _keeps_region
+
+    return _keeps_region(M, N, split)
+
+
 def work(name: str, B, H, Hk, M, N, D, causal, split, elem=2):
     """(algorithmic FLOP, algorithmic HBM bytes) of one call."""
     ep, _, _, fac = WORKLOADS[name]
@@ -113,7 +122,7 @@ def work(name: str, B, H, Hk, M, N, D, causal, split, elem=2):
     Px = cross_pairs(M, N, split, causal, off)
     if name == "cross_qk":
         return 4 * B * H * D * P, qkvo + 4 * B * Hk * split
-    if name == "cross_softmax":
+    if name == "cross_softmax" or not keeps_region(M, N, split):
         return 4 * B * H * D * P + 2 * B * H * D * Px, qkvo + 4 * B * Hk * split
     # buffered: pass 2 reloads the region instead of recomputing its scores.
     # The region leaves pass 1 as fp16 exponents (2 bytes a score) plus one

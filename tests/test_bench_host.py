@@ -54,6 +54,19 @@ def test_every_workload_has_a_model(name):
     assert nbytes >= 2 * (2 * 2 * 8 * 256 * 64 + 2 * 2 * 4 * 384 * 64)
 
 
+def test_buffered_sum_is_charged_for_what_runs():
+    """A large region is recomputed: cross_softmax's work, not two passes over a
+    region in memory.  A small one is written and read once."""
+    large = (1, 32, 8, 4096, 4096, 128, True, 3072)
+    assert bench.work("cross_softmax_buffered", *large) == bench.work("cross_softmax", *large)
+    small = (1, 4, 4, 296, 296, 128, True, 256)
+    flop, nbytes = bench.work("cross_softmax_buffered", *small)
+    region = 4 * (296 - 256) * (2 * 256 + 4 * 4)
+    assert nbytes == bench.work("cross_softmax", *small)[1] + 2 * region
+    assert flop < bench.work("cross_softmax", *small)[0]
+    assert bench.WORKLOADS["cross_softmax_buffered"][2] == "mfma"
+
+
 def test_backward_is_two_and_a_half_forwards():
     f, _ = bench.work("attention_fwd", 1, 4, 4, 128, 128, 64, True, None)
     b, _ = bench.work("attention_bwd", 1, 4, 4, 128, 128, 64, True, None)
