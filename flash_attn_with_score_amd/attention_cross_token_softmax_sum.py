@@ -15,8 +15,8 @@ __all__ = ["attention_cross_token_softmax_sum", "attention_cross_token_softmax_s
 
 # The buffered variant keeps the region's scores only where that is faster than
 # a second pass over K: at most BUFFERED_ROWS query rows past the split over at
-# most BUFFERED_KEYS keys whose region rows start on 16 bytes, or twice the rows
-# at any split over at most BUFFERED_SHORT keys.  Time kept / recomputed, mean over six head
+# most BUFFERED_KEYS keys whose region rows start on 16 bytes, or at any split
+# over at most BUFFERED_SHORT keys.  Time kept / recomputed, mean over six head
 # counts and D = 32, 64, 128 (fp16, causal), 64 rows: S 200 0.96, 296 0.95, 384
 # 0.90, 448 1.00, 512 1.04; 8 rows 0.83, 0.82, 0.83, 0.92, 0.97; 128 rows 1.02
 # to 1.09; splits that are no multiple of 8, 33 rows: S 136 0.91, 200 1.08, 296
@@ -25,9 +25,8 @@ BUFFERED_ROWS, BUFFERED_KEYS, BUFFERED_SHORT = 64, 448, 160
 
 
 def _keeps_region(M: int, N: int, split: int) -> bool:
-    if N <= BUFFERED_SHORT:
-        return M - split <= 2 * BUFFERED_ROWS
-    return M - split <= BUFFERED_ROWS and N <= BUFFERED_KEYS and split % 8 == 0
+    keys = BUFFERED_KEYS if split % 8 == 0 else BUFFERED_SHORT
+    return M - split <= BUFFERED_ROWS and N <= keys
 
 
 def attention_cross_token_softmax_sum_buffered(

@@ -465,7 +465,7 @@ def test_make_args_packs_every_field():
 
 @pytest.mark.parametrize("M,N,split,kept", [
     (448, 448, 384, True), (448, 448, 376, False), (456, 456, 400, False),
-    (400, 400, 341, False), (400, 400, 344, True), (160, 160, 33, True), (160, 160, 31, False),
+    (400, 400, 341, False), (400, 400, 344, True), (160, 160, 97, True), (160, 160, 95, False),
     (161, 161, 133, False),
     (40, 168, 8, True), (8, 400, 40, True)])
 def test_buffered_sum_keeps_small_regions(M, N, split, kept):
