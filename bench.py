@@ -1,6 +1,6 @@
 """Benchmark of the fused attention family on one MI355X.
 
-Default workload (the shape BASELINE.json's metric is quoted on):
+Default workload (the shape the headline metric is quoted on):
 attention_with_scores, B=1, H=32, M=N=4096, D=128, fp16, causal.  A "step"
 is one call of the drop-in entry point over that batch with q/k/v already
 resident in HBM.  The line printed is the driver's JSON contract plus

@@ -254,20 +254,22 @@ __device__ __forceinline__ int64_t* region_rows() {
 // per-lane head offset folds away at compile time.
 // The 4-wave score writer (64-row blocks) runs one wave per SIMD (its LDS:
 // one workgroup per CU), the others two, or four (fwd_waves).
-// KS2 (unpacked score writer): row blocks of 32 * NW / 2 rows whose key
-// range is split between the wave pairs: loader wave i takes the even key
-// tiles and storer wave NW/2 + i the odd ones of the same 32 rows, so a step
-// stages two key tiles; at the end each storer hands its partial O, offset
-// and weight sum to its loader through LDS.  For problems whose 128-row
-// blocks all run in one round, where the longest causal row block alone set
-// the kernel time:
-//  * 4 waves, 64-row blocks: two rounds whose longest-first pairs (rb,
-//    15 - rb) all take the same number of steps (one wave per SIMD);
+// KS2 (the unpacked score writer, and the plain and row-sum modes, packed or
+// with dropout too): row blocks of 32 * NW / 2 rows whose key range is split
+// between the wave pairs: wave i (the writer's loader) takes the even key tiles
+// and wave NW/2 + i (its storer) the odd ones of the same 32 rows, so a step
+// stages two key tiles; at the end the upper wave hands its partial O, offset,
+// weight sum and row sum to the lower one through LDS.  For problems of one or
+// two rounds of row blocks, whose longest causal block sets the kernel time
+// (fwd_plan and attention_with_scores_impl choose):
+//  * 4 waves, 64-row blocks (score writer): one round, or two whose
+//    longest-first pairs (rb, 15 - rb) all take the same number of steps (one
+//    wave per SIMD);
 //  * 8 waves, 128-row blocks: two waves per SIMD, half the steps of the
-//    256-row writer per row block.  Its K/V stages fill 128 KiB
-//    of LDS, so the loaders' score tiles are single-buffered: a second
-//    barrier in each step (after the tiles are staged) hands them to the
-//    storers, which store both tiles of the step during O += P V.
+//    256-row blocks.  The writer's K/V stages fill 128 KiB of LDS, so the
+//    loaders' score tiles are single-buffered: a second barrier in each step
+//    (after the tiles are staged) hands them to the storers, which store both
+//    tiles of the step during O += P V.
 // ALN (score writer): whether the score rows start on 64-byte boundaries
 // (store_score16).
 // Waves per SIMD (two workgroups a CU for four): up to D = 32 the step is the
@@ -1357,8 +1359,8 @@ __global__ __launch_bounds__(256) void fwd_combine_kernel(const FwdParams p) {
 
 // Second pass of kFwdFewRows: col[key] = sum over the G*M rows of a KV head of
 // exp2(s * qk_scale - lse2), from the scores the forward kept (4 G M bytes a
-// key where a pass over K reads 2 D: B8 H32/8 M1 N8191 D128, 98 us with the
-// column pass over K, 8 us here).  With a key split, workgroups
+// key where a pass over K reads 2 D: B8 H32/8 M1 N8191 D128, 98 us for the
+// column pass over K and 5 to merge the splits, 5.6 us for both here).  With a key split, workgroups
 // [0, ncombine) merge the output rows as fwd_combine_kernel does and the
 // others form the base-2 normalizers themselves, 8 threads a row, so one
 // launch follows the forward.  A workgroup sums 1024 keys, four a thread.

@@ -81,7 +81,8 @@ struct FwdParams {
   int pack;
   int pack_shift;    // log2(pack) when pack is 1, 2, 4 or 8 (the score writer's packings)
   int nrb;           // virtual row blocks per group of `pack` heads
-  int bm;            // rows per workgroup (256, the score writer also 128 or 64)
+  int bm;            // rows per workgroup: 256; 128 in the plain, row-sum and score modes, 64
+                     // in the score writer
   int scores_aligned;  // score rows start on 64-byte boundaries and N % 8 == 0
   int zero_self;     // score writer: 1 = a workgroup writes its own row block's zeros
                      // (all workgroups run at once), 0 = its mirror row block's

@@ -1,4 +1,4 @@
-"""GPU parity at the BASELINE.json configurations (full sizes).
+"""GPU parity at the benchmark configurations (full sizes).
 
 At these sizes the CPU oracle runs on a bounded part of the problem (one KV
 group, or a block of query rows) and the rest is checked through properties
@@ -13,8 +13,8 @@ that hold at any size:
     atomic order), bit for bit;
   * the stored (rounded) scores' row sums match the row-sum entry point.
 
-Configs (BASELINE.json "configs"): 2 is covered by test_gpu_parity.py; 3, 4
-and 5 are here.  Inputs follow oracle/inputs.py (seed 0, CPU generator).
+Configuration 2 (B1 H32 S1024) is covered by test_gpu_parity.py; 3, 4 and 5
+are here.  Inputs follow oracle/inputs.py (seed 0, CPU generator).
 """
 from __future__ import annotations
 
@@ -144,7 +144,7 @@ def test_metric_shape_scores_properties(gpu):
 
 
 def test_metric_shape_softmax_col_sum(gpu):
-    """The north star's MFMA target, attention_with_softmax_col_sum at
+    """attention_with_softmax_col_sum at the metric shape,
     B1 H32 S4096 D128 fp16 causal (attention_with_col_softmax_sum.py:224-270):
     three heads against the oracle, and for every head the column sums add up
     to S (each of the S softmax rows sums to 1)."""
