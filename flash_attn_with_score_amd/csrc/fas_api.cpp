@@ -499,11 +499,14 @@ struct FwdPlan {
 //  * steps of the 128-row blocks move twice the K/V bytes per row, and a chip
 //    that runs evenly loaded clocks lower than one waiting for its longest
 //    row blocks: they count 1.2.  Up to 128 rows a 256-row block has one wave
-//    per SIMD and the pairs two: 1.5, and 1.8 with dropout, whose step (about
-//    3 us) is the VALU's;
-//  * a key split adds the combine kernel: about 6 us, 0.1 us a split (a row's
-//    splits are merged one after the other), and its partials written and
-//    read back at 5 TB/s.
+//    per SIMD and the pairs two: 1.5.  Dropout's step (2 to 3 us) is the
+//    VALU's: 1.1, and up to 128 rows 1.35, but 1.8 against a split;
+//  * a key split adds the combine kernel: about 5 us, 1 us for every eight
+//    splits (whose loads a row keeps in flight together) and 0.6 for each of
+//    the rest, and its partials written and read back at 5 TB/s.  Splits past
+//    a causal row block's last key end at once: with dropout, whose steps are
+//    the long ones, they start no round (B1 H16 S1531 D16 in three, 288
+//    workgroups of which 192 have keys: 41 us, as pairs 50).
 // Fitted to 1255 timed calls; the choice taken is 1.5% above the fastest in
 // the mean.  Measured (us, row-sum calls; 256 rows / 128 rows /
 // split): B1 H32 S1024 D128 causal 34.3 / 24.1; S2048 59.9 / 49.2; S4096 147 /
@@ -512,22 +515,18 @@ struct FwdPlan {
 // 111 / 45.4 in eight (61.2 in 14, two rounds); B1 H8/1 M4 N32768 D16, in 32 /
 // 64 / 256: 21 / 22 / 47; B8 H32/8 M1 N32768 D16 in 4 / 8 (two a CU): 75 / 45;
 // dropout 0.1, B1 H32 M128 N1024 D64: 44 / 40 / 30 in two.
-// attention() (lse_out) also returns the log-normalizer, the same bits with and
-// without dropout for one query head per KV head (D <= 32: up to one workgroup
-// a CU): up to 128 rows all its calls take dropout's choice, above that none.
 FwdPlan fwd_plan(const Problem& pr, int pack, bool top_left, const SplitPlan& cap,
-                 bool key_pairs, bool lse_out) {
+                 bool key_pairs) {
   FwdPlan best;
   const int64_t cus = kCus, groups = (int64_t)pr.B * (pr.H / pack);
   const int64_t rows = (int64_t)pr.M * pack, n256 = groups * ((rows + 255) / 256);
   if (n256 == 0 || pr.N == 0 || n256 > 2 * cus) return best;
   const int64_t off = top_left ? 0 : (int64_t)pr.N - pr.M;
   const bool few = (int64_t)pr.G * pr.M <= kFewRows;
-  const bool two = pr.D <= 32 && !pr.dropout;  // workgroups per CU
   const double share = few ? 1.3 : 1.5;
   const bool half = rows <= 128;
-  const bool drop_half = !few && (pr.dropout || lse_out) && pr.M <= 128;
-  const bool drop_full = !few && pr.dropout && !lse_out && pr.M > 128;
+  const bool drop_half = !few && pr.dropout && half, drop_full = !few && pr.dropout && !half;
+  const bool two = pr.D <= 32 && !pr.dropout;  // workgroups per CU
   // Steps of row block rb: its key tiles, or pairs of them.
   auto steps = [&](int64_t bm, int64_t rb) {
     int64_t hi = pr.N;
@@ -551,25 +550,42 @@ FwdPlan fwd_plan(const Problem& pr, int pack, bool top_left, const SplitPlan& ca
   double cost = makespan(256, 2.5);
   if (key_pairs && n256 <= cus) {
     const double c =
-        (drop_half ? 1.8 : drop_full ? 1.1 : half || few ? 1.5 : 1.2) * makespan(128, 3.0);
+        (drop_half ? 1.35 : drop_full ? 1.1 : half || few ? 1.5 : 1.2) *
+        makespan(128, 3.0);
     if (c < cost) {
-      cost = c;
+      // (Against 256 rows on the same CU; a split takes other CUs.)
+      cost = drop_half ? 1.8 / 1.35 * c : c;
       best.bm = 128;
     }
   }
   const int64_t nt = steps(256, (rows + 255) / 256 - 1);
-  const double us_per_step = drop_half ? 2.0 : drop_full ? 3.0 : few ? (pr.D == 128 ? 1.0 : 0.7)
+  // Workgroups that have key tiles, as if every XCD had as many as the one that
+  // has most (consecutive workgroups, the splits of a row block, go to
+  // consecutive XCDs), and a fifth more: they are not spread evenly within one
+  // (B1 H1 M4096 N16384 D64 dropout, 252 of 288 in 18 splits: 173 us, 16: 123).
+  auto busy = [&](int64_t ns, int64_t tps) {
+    const int64_t g = ns % 8 == 0 ? 8 : ns % 4 == 0 ? 4 : ns % 2 == 0 ? 2 : 1;
+    int64_t first = 0;  // splits 0, g, 2 g, ... with tiles
+    for (int64_t rb = 0; rb < (rows + 255) / 256; ++rb)
+      first += ((steps(256, rb) + tps - 1) / tps + g - 1) / g;
+    return std::min(n256 * ns, first * g * groups * 6 / 5);
+  };
+  const double us_per_step = drop_half   ? 2.0
+                             : drop_full ? 3.0
+                             : few       ? (pr.D == 128 ? 1.0 : 0.7)
                              : pr.D == 128 ? 1.7 : 1.0;
   for (int64_t want = 2; want <= cap.nsplit; ++want) {
     const int64_t tps = (nt + want - 1) / want, ns = tps > 0 ? (nt + tps - 1) / tps : 0;
     if (ns != want) continue;
     const int64_t n = n256 * ns;
-    const double rounds = !two       ? (double)((n + cus - 1) / cus)
-                          : n <= cus ? 1.0
-                                     : share * (double)((n + 2 * cus - 1) / (2 * cus));
+    const double rounds = n <= cus ? 1.0
+                          : two    ? share * (double)((n + 2 * cus - 1) / (2 * cus))
+                          : drop_full && pr.causal
+                              ? (double)((busy(ns, tps) + cus - 1) / cus)
+                              : (double)((n + cus - 1) / cus);
     const double partials = (double)pr.B * pr.H * pr.M * (double)ns * (pr.D + 3) * 8;
-    const double c =
-        rounds * ((double)tps + 2.5) + (6.0 + 0.1 * (double)ns + partials / 5e6) / us_per_step;
+    const double merge = 5.0 + (double)(ns / 8) + 0.6 * (double)(ns % 8);
+    const double c = rounds * ((double)tps + 2.5) + (merge + partials / 5e6) / us_per_step;
     if (c < cost) {
       cost = c;
       best.bm = 256;
@@ -742,7 +758,7 @@ Workspace layout(int variant, const Problem& pr, int64_t split, size_t budget = 
     if (variant == FAS_VARIANT_SOFTMAX_COL_SUM && few_rows(pr)) {
       const size_t bytes =
           align256((size_t)pr.B * pr.H * pr.M * (((size_t)pr.N + 63) / 64 * 64) * 4);
-      const int want = fwd_plan(pr, pr.pack, false, split_plan(pr, false), false, false).nsplit;
+      const int want = fwd_plan(pr, pr.pack, false, split_plan(pr, false), false).nsplit;
       if (bytes <= kFewMaxBytes && off + bytes <= budget &&
           2 * split_plan(pr, false, 255, budget - off - bytes).nsplit >= want) {
         w.has_few = true;
@@ -872,8 +888,8 @@ T* at(void* ws, size_t off) {
 
 // Row blocks and key split of a plain or row-sum forward, with its partials.
 void apply_plan(fas::FwdParams& p, const Problem& pr, bool top_left, const Workspace& w, void* ws,
-                bool key_pairs = true, bool lse_out = false) {
-  const FwdPlan f = fwd_plan(pr, p.pack, top_left, w.sp, key_pairs, lse_out);
+                bool key_pairs = true) {
+  const FwdPlan f = fwd_plan(pr, p.pack, top_left, w.sp, key_pairs);
   p.bm = f.bm;
   p.nrb = (int)(((int64_t)pr.M * p.pack + f.bm - 1) / f.bm);
   if (f.nsplit == 1) return;
@@ -1400,7 +1416,7 @@ int fas_attention_forward(const fas_attn_args* a, float* lse, const int64_t st[3
   if ((rc = check_keep(fn, a, pr, &kl))) return rc;
   fas::FwdParams p = fwd_params(a, pr, false, fas::kFwdRows);
   rescale_dropout(p, a);
-  apply_plan(p, pr, false, w, ws, true, true);
+  apply_plan(p, pr, false, w, ws);
   p.lse_ln = lse;
   p.sl0 = st[0];
   p.sl1 = st[1];
