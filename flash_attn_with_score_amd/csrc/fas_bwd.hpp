@@ -159,8 +159,9 @@ void bwd_dkdv_kernel(const BwdParams p) {
   const int rstart = p.causal ? max(0, kb * BK - p.causal_off) : 0;
   const int tlo = rstart / TQ, tiles = max(0, (p.M + TQ - 1) / TQ - tlo);
   // This piece's tiles [s0, s1) of the G heads' tiles in head order.
-  const int64_t steps = (int64_t)p.G * tiles;
-  const int s0 = (int)(steps * piece / p.pieces), s1 = (int)(steps * (piece + 1) / p.pieces);
+  int s0, s1;
+  deal(p.G * tiles, piece, p.pieces, s0, s1);
+  s1 += s0;
   const float qk = p.qk_scale;
   const uint32_t q_base = lds_addr(&qlds[0][0]), g_base = lds_addr(&glds[0][0]);
 

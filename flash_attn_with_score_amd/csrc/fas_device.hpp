@@ -256,6 +256,14 @@ __device__ __forceinline__ void store_score_tail(u32x4 v, __amdgpu_buffer_rsrc_t
                                             off + 2u * (uint32_t)e, soff, 0);
 }
 
+// Part i of n nearly equal runs of `steps` (the first ones one longer): its
+// first step and its length.
+__device__ __forceinline__ void deal(int steps, int i, int n, int& first, int& count) {
+  const int q = steps / n, r = steps - q * n;
+  first = q * i + (i < r ? i : r);
+  count = q + (i < r ? 1 : 0);
+}
+
 // a ^ b ^ c in one instruction (v_bitop3_b32; 0x96 is the truth table of the
 // three-way exclusive or over operand bytes 0xF0, 0xCC, 0xAA).
 __device__ __forceinline__ uint32_t xor3(uint32_t a, uint32_t b, uint32_t c) {

@@ -259,8 +259,9 @@ void colsm64_kernel(const ColsmParams p) {
     const int t0 = max(0, rstart) / TQ;
     const int nt = t1 > t0 ? t1 - t0 : 0;
     // This split's share of the block's (head, step) pairs, head-major.
-    const int first = (int)((int64_t)p.fold * nt * item.sp / p.nsplit);
-    const int nsteps = (int)((int64_t)p.fold * nt * (item.sp + 1) / p.nsplit) - first;
+    // (32-bit division: a 64-bit one costs a short launch 1 us.)
+    int first = 0, nsteps = p.fold * nt;
+    if (p.nsplit > 1) deal(nsteps, item.sp, p.nsplit, first, nsteps);
 
     float colacc[2] = {0.f, 0.f};
     // Keep words of step t of head h (DROP == 2): block (qb, j) is rows
