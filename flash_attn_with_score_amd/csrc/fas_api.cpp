@@ -643,8 +643,14 @@ int bwd_pieces(const Problem& pr) {
     if (s > 1 && tiles(0) < 4 * s) break;
     const double longest = (double)((tiles(0) + s - 1) / s) + 3.0;
     double c = std::max(longest, (sum + 3.0 * (double)(n * s)) / (double)slots);
-    // Blocks of equal length run in whole rounds.
-    if (!pr.causal) c = longest * (double)((n * s + slots - 1) / slots);
+    // Blocks of equal length run in whole rounds; of two rounds of others the
+    // last of the first and the first of the second may end last.
+    if (!pr.causal) {
+      c = longest * (double)((n * s + slots - 1) / slots);
+    } else if (n * s > slots && n * s <= 2 * slots) {
+      auto at = [&](int64_t i) { return (double)((tiles(i / (heads * s)) + s - 1) / s) + 3.0; };
+      c = std::max(c, at(slots - 1) + at(slots));
+    }
     if (s > 1)
       c += (6.0 + (double)heads * pr.N * s * 2 * pr.D * 8 / 5e6) / us_per_tile;
     if (c < cost) {
