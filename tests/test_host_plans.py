@@ -267,3 +267,43 @@ def test_kept_scores_stay_below_4_gib(lib):
         assert launches(lib, "softmax_col_sum", a)[0][1]["kept"] == kept
     nbytes = lib.fas_workspace_bytes(_native.VARIANT_SOFTMAX_COL_SUM, ctypes.byref(a), 0)
     assert nbytes < 1 << 30
+
+
+@pytest.mark.parametrize("seed", range(3))
+def test_planned_launches_are_taken(lib, seed):
+    """Random requests: every planned launch is one that its launcher takes (the
+    row blocks, packings and splits that have instances), also from workspaces
+    for one head at a time and with unaligned score rows."""
+    rng = random.Random(100 + seed)
+    for _ in range(400):
+        Hk, G = rng.choice([1, 1, 2, 3, 8, 32]), rng.choice([1, 1, 2, 3, 4, 7, 8, 16, 32, 64])
+        M = rng.choice([1, 2, 5, 32, 33, rng.randint(1, 300), rng.randint(1, 5000)])
+        N = rng.choice([1, 63, 64, rng.randint(1, 1200), rng.randint(1, 40000)])
+        B, D = rng.choice([1, 1, 2, 16, 64]), rng.choice([16, 32, 64, 128])
+        causal, dropout = rng.choice([0, 1]), rng.choice([0.0, 0.0, 0.2])
+        entry = rng.choice(["scores", "scores", "row_sum", "softmax_col_sum", "attention_forward",
+                            "attention_backward", "cross_softmax_sum"])
+        split = rng.randint(1, N) if entry == "cross_softmax_sum" else 0
+        a = make_args(B, Hk * G, Hk, M, N, D, causal, dropout)
+        case = (entry, B, Hk * G, Hk, M, N, D, causal, dropout, split)
+        for name, f in launches(lib, entry, a, split):
+            if name == "fwd":
+                assert f["nsplit"] >= 1 and f["nrb"] == -(-M * f["pack"] // f["bm"]), case
+                assert f["pack"] == 1 or not dropout, case
+                if f["nsplit"] > 1:
+                    assert f["bm"] == 256 and f["mode"] != SCORES, case
+                    assert (f["nsplit"] - 1) * f["tps"] < -(-N // 64) <= f["nsplit"] * f["tps"], case
+                if f["mode"] == SCORES:
+                    assert f["bm"] == 256 or (f["bm"] in (64, 128) and f["pack"] == 1
+                                              and not dropout), case
+                elif f["bm"] != 256:
+                    assert f["bm"] == 128 and f["mode"] in (PLAIN, ROWSUM, 4), case
+                if f["mode"] == FEW:
+                    assert f["pack"] == G and G * M <= 32 and not dropout and f["bm"] == 256, case
+            elif name == "scores" and f["ngrp"] > 0:
+                assert f["ngrp"] <= f["nkb"] and f["pshift"] <= 3, case
+                assert G % (1 << f["pshift"]) == 0 and M << f["pshift"] <= 512, case
+            elif name == "colsm":
+                assert 1 <= f["nsplit"] <= 8 * G, case
+            elif name == "bwd":
+                assert 1 <= f["pieces"] <= max(8, G), case
