@@ -429,11 +429,15 @@ bool few_rows(const Problem& pr) {
 //  * other shapes: 24 from 3000 keys on (H1 M512 N3000 D128 44 / 54, H12 35 /
 //    39 with D64; H4 M2048 N2048 46 / 38), 32 from 4096 (H1 S4096 47 / 64, H12
 //    M700 56 / 68; H12 M1024 71 / 63), 64 from 16384 (H4 M4096 234 / 264);
-//  * up to 128 rows over 1536 to 2047 keys, D >= 64: 32 (H1 M48 N1536 D128 24 /
-//    29, H12 M100 N1600 27 / 31; D32 21 / 20, N1024 24 / 22);
-//  * few rows of so many heads that even the 64-row blocks need a second round
-//    (a KV head's heads share a workgroup here, not there): every row block,
-//    from 16 key tiles on (B64 H32/1 M1 N1000 D64 134 / 171).
+//  * up to 128 rows of a KV head, 32, below 2048 keys: from 1280 at D = 128,
+//    1400 at 64, 1800 below (H1 M48 N1536 D128 24 / 29, H12 M100 N1600 27 / 31;
+//    D32 21 / 20, D128 N1024 24 / 22);
+//  * few rows, whose forward writes the scores itself (kFwdFewRows), 128, below
+//    2048 keys: from 961 at D = 128, 1281 below (H4 M1 N1500 D128 18 / 32, D16 18
+//    / 21, N1024 D16 18 / 14; B8 H32/8 M1 N2000 D128 22 / 39; with 192 row blocks
+//    B16 H12 M2 N2000 D128 45 / 41); and every row block of so many heads that
+//    even the fused writer's 64-row blocks need a second round (a KV head's heads
+//    share a workgroup here, not there; B64 H32/1 M1 N1000 D64 30 / 171).
 // With dropout the fused writer has 256-row blocks only and its step is the
 // random stream's products, which a split spreads over the CUs: up to 64 row
 // blocks whatever the keys (split / fused with dropout 0.1: B1 H1 S4096 D64 57
@@ -442,8 +446,10 @@ static int64_t scores_split_max_wgs(const Problem& pr) {
   const int64_t m = pr.M, n = pr.N;
   if (pr.dropout) return n >= 64 * m ? 256 : n >= 8 * m ? 128 : 64;
   if (few_rows(pr) && n > 960 && (int64_t)pr.B * pr.H * ((m + 63) / 64) > kCus) return 256;
-  if (n < 2048)
-    return n >= 1536 && n >= 8 * m && pr.D >= 64 && (int64_t)pr.G * m <= 128 ? 32 : 0;
+  if (n < 2048) {
+    if (few_rows(pr)) return n > (pr.D == 128 ? 960 : 1280) ? 128 : 0;
+    return (int64_t)pr.G * m <= 128 && n >= (pr.D == 128 ? 1280 : pr.D == 64 ? 1400 : 1800) ? 32 : 0;
+  }
   if (n >= 8 * m) return n >= 64 * m ? 256 : 128;
   return n >= 16384 ? 64 : n >= 4096 ? 32 : n >= 3000 ? 24 : 0;
 }
@@ -760,7 +766,9 @@ Workspace layout(int variant, const Problem& pr, int64_t split, size_t budget = 
     // budget leaves the key split half the splits the forward would take: one
     // with fewer costs what the column pass over K does (B8 H32/8 M1 N32768
     // D128, four splits: 250 us, in two 329, unsplit 556; the pass over K 590)
-    // and more where few row blocks need many splits.
+    // and more where few row blocks need many splits.  (Kept / the pass over
+    // K, us: B8 H32/8 M8 N8192 D64 48 / 102, B64 H32/1 M1 N4100 D16 28 / 240, H32
+    // M32 N32768 D16 64 / 86, D32 103 / 93, D128 179 / 227.)
     if (variant == FAS_VARIANT_SOFTMAX_COL_SUM && few_rows(pr)) {
       const size_t bytes =
           align256((size_t)pr.B * pr.H * pr.M * (((size_t)pr.N + 63) / 64 * 64) * 4);
@@ -1225,7 +1233,9 @@ static int attention_with_scores_impl(const fas_attn_args* a, void* scores, cons
     fas::FwdParams p = fwd_params(a, pr, false, fas::kFwdRows);
     rescale_dropout(p, a);
     if (few_rows(pr)) {
-      // The forward writes the scores itself: K is read once.
+      // The forward writes the scores itself: K is read once (us, key-split
+      // forward and scores kernel / here: B8 H32/8 M1 N32768 D128 304 / 229, D16
+      // 86 / 65; B16 H12 M2 N8192 D64 148 / 139; H32 M32 N32768 D64 89 / 79).
       apply_plan(p, pr, false, w, ws, false);
       p.scores = static_cast<uint16_t*>(scores);
       p.ss0 = st[0]; p.ss1 = st[1]; p.ss2 = st[2];

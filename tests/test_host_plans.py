@@ -132,8 +132,15 @@ SCORES_PLANS = [
     ((1, 4, 4, 2048, 2048, 128), SCORES, 64),    # 32 over 2048: fused
     ((1, 12, 12, 1024, 4096, 64), SCORES, 64),   # 48 over 4096
     ((1, 4, 4, 4096, 16384, 128), PLAIN, None),  # 64 over 16384
-    ((2, 12, 12, 48, 1600, 128), PLAIN, None),   # few rows over 1536 keys and more
+    ((2, 12, 12, 48, 1300, 128), PLAIN, None),   # up to 128 rows below 2048 keys
+    ((2, 12, 12, 48, 1600, 64), PLAIN, None),
     ((2, 12, 12, 48, 1600, 32), SCORES, 64),
+    ((2, 12, 12, 48, 1900, 32), PLAIN, None),
+    ((2, 12, 12, 160, 1900, 128), SCORES, 64),
+    ((1, 4, 4, 1, 1000, 128), FEW, None),        # few rows below 2048 keys
+    ((1, 4, 4, 1, 1024, 64), SCORES, 64),
+    ((1, 8, 1, 4, 1300, 16), FEW, None),
+    ((16, 12, 12, 2, 2000, 128), SCORES, 64),    # 192 row blocks
     ((2, 12, 12, 48, 1024, 128), SCORES, 64),
     ((64, 32, 1, 1, 1000, 64), FEW, None),       # 2048 heads: the fused writer needs 8 rounds
     ((64, 32, 1, 1, 960, 64), SCORES, 256),
